@@ -638,7 +638,7 @@ def pmc_workload(ctx, launches, which="gemv"):
         f"bytes, 4 copies of {src.numel() * 4} bytes")
 
 
-STAGE_PHASES = ("mfma_decode", "store_issue", "a_wait", "barrier")
+STAGE_PHASES = ("multiply", "multiply_barrier", "decode", "decode_barrier")
 CLOCK_LIB = ROOT / "strix-trellis_amd" / "strix_trellis" / "_native" / "libstrix_trellis_clock.so"
 
 

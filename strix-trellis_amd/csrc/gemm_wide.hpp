@@ -88,11 +88,12 @@ constexpr uint32_t kHandoffForceRecompute = 0xFFFFFFFFu;   // poll_limit: always
 
 // Phase clock of one wave (s_memtime, shader clock cycles), compiled in only
 // by the instrumented build (STX_STAGE_CLOCK=1, build.py --stage-clock); in
-// the product build every member is empty.  Per K stage the loop is cut into
-//   0: MFMAs of stage st with the interleaved decode of stage st + 1,
-//   1: the decoded B fragments to LDS and the next chunk loads issued,
-//   2: the wait for A stage st + 1 (vmcnt),
-//   3: the stage barrier;
+// the product build every member is empty.  Per K stage a wave's loop is cut into
+//   0: M, the stage's MFMAs,
+//   1: the barrier that ends M's slot,
+//   2: D up to its chunk loads: A DMAs issued, the other stage's blocks decoded
+//      into LDS, the next chunk loads issued,
+//   3: the rest of D: the next fragments read, the A wait and the barrier;
 // scheduling barriers pin each mark, so the instrumented loop keeps these
 // phases in this order.  A record is 16 words per wave:
 //   [phase 0..3 sums][prologue][epilogue][t0][realtime0][t1][realtime1]
@@ -173,9 +174,11 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
     const uint32_t row_bytes = (N >> 4) * tile_bytes;
     const auto wrsrc = make_rsrc(a.trellis, uint32_t(uint64_t(I / 16) * row_bytes));
     const auto arsrc = make_rsrc(a.afrag, uint32_t(a.afrag_bytes));
-    constexpr int kDecoders = NT * 4 / 8;                // wave units of 8 tiles x 1 block
-    const bool decoder = BN == 256 || w < kDecoders;
-    const int dblk = BN == 256 ? w >> 1 : w & 3;         // decode role
+    // Waves 0-3 (the early half, one per SIMD) decode the last two input blocks
+    // of a stage, waves 4-7 (the late half) the first two (see the K loop).
+    const int late = w >> 2;
+    const bool decoder = BN == 256 || (w & 3) < 2;
+    const int dblk = BN == 256 ? (w >> 1) ^ 2 : (late ? w & 1 : 2 + (w & 1));
     const int dtile = BN == 256 ? 8 * (w & 1) + jt8 : jt8;
 
     // XCD-aware tile order: workgroup i runs on XCD i % 8 (round-robin
@@ -246,9 +249,8 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
         __syncthreads();   // every wave has read it before the prologue's DMAs reuse the word
     }
 
-    // ---- B: chunk ring (stage st in slot st % D), one chunk per lane ----
-    constexpr int D = 1;   // chunk ring depth; 2 would spill at 256 VGPRs
-    Chunk<K> ring[D];
+    // ---- B: one chunk of the next stage to decode, one chunk per lane ----
+    Chunk<K> chunk;
     // The stage's part of the offset is a scalar operand.  Past the end, or for
     // a wave that does not decode, the lane offset itself goes out of range:
     // the buffer range check covers the vector and immediate offsets, not the
@@ -261,48 +263,53 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
     // input block dblk: column n = 16 (dtile % 2) + g (+8) of 32-column block
     // dtile / 2; rows 0..7 go to fragment lane n, rows 8..15 to lane 32 + n
     // (the A-operand order A[n][k]).
-    auto store_bfrag = [&](const half2_t (&wq)[4][4], int buf) {
-        unsigned char* base = bbuf + buf * WIDE_TILE_BYTES + ((dtile >> 1) * 4 + dblk) * 1024;
-        const int n = 16 * (dtile & 1) + g;
-        auto frag = [&](int l) -> u32x4* { return reinterpret_cast<u32x4*>(base + l * 16); };
-        *frag(n) = u32x4{as_u32(wq[0][0]), as_u32(wq[1][0]), as_u32(wq[2][0]), as_u32(wq[3][0])};
-        *frag(32 + n) = u32x4{as_u32(wq[0][1]), as_u32(wq[1][1]), as_u32(wq[2][1]), as_u32(wq[3][1])};
-        *frag(n + 8) = u32x4{as_u32(wq[0][2]), as_u32(wq[1][2]), as_u32(wq[2][2]), as_u32(wq[3][2])};
-        *frag(40 + n) = u32x4{as_u32(wq[0][3]), as_u32(wq[1][3]), as_u32(wq[2][3]), as_u32(wq[3][3])};
-    };
+    // The four fragment words of one (column half h, row half k) leave the
+    // decoder as plain registers: a [4][4] array of pairs turned into 16-byte
+    // vectors went through scratch memory.
     auto decode_stage = [&](Chunk<K>& src, int buf) {
         if (!decoder) return;
         link_chunk(src, g == 0);
-        half2_t wq[4][4];
-        decode_chunk<K, CB>(src, wq);
-        store_bfrag(wq, buf);
+        unsigned char* base = bbuf + buf * WIDE_TILE_BYTES + ((dtile >> 1) * 4 + dblk) * 1024;
+        const int n = 16 * (dtile & 1) + g;
+        auto frag = [&](auto fc, int l) {
+            constexpr int F = decltype(fc)::value;
+            const uint32_t f0 = as_u32(decode_pair<K, CB, 0, F>(src)), f1 = as_u32(decode_pair<K, CB, 1, F>(src));
+            const uint32_t f2 = as_u32(decode_pair<K, CB, 2, F>(src)), f3 = as_u32(decode_pair<K, CB, 3, F>(src));
+            *reinterpret_cast<u32x4*>(base + l * 16) = u32x4{f0, f1, f2, f3};
+        };
+        frag(std::integral_constant<int, 0>{}, n);
+        frag(std::integral_constant<int, 2>{}, 32 + n);
+        frag(std::integral_constant<int, 4>{}, n + 8);
+        frag(std::integral_constant<int, 6>{}, 40 + n);
     };
 
-    // ---- A: wave w DMAs fragments 4w..4w+3 (fragment f = 32-row block f/4,
-    // K16 step f%4) of a stage straight into LDS (buffer_load ... lds).  Three
-    // A buffers: stage st is issued two stages ahead, into buffer st % 3.
-    // Lane part of the fragment offsets (row block 8 mb + w); the stage's K
-    // part is a scalar operand (always in range), and K16 step q the
-    // immediate offset q * 1 KiB, which the load adds to both the memory and
-    // the LDS address.
-    const uint32_t a_voff = uint32_t(afrag32_offset(uint32_t(mb) * 8 + w, 0, I, lane));
+    // ---- A: fragment f of a stage is 32-row block f / 4, K16 step f % 4.  Each
+    // half DMAs (buffer_load ... lds) the K16 steps whose weights it decodes,
+    // wave w those of row blocks 2 (w % 4) and 2 (w % 4) + 1.  Three A buffers
+    // (stage st in buffer st % 3).  The row-block part of the offset is the
+    // lane's, the stage's K part a scalar operand (always in range), and the
+    // K16 step the immediate offset q * 1 KiB, which the load adds to both the
+    // memory and the LDS address.
+    const uint32_t a_rb = 2u * (w & 3), a_k0 = late ? 0u : 2u;
+    const uint32_t a_voff0 = uint32_t(afrag32_offset(uint32_t(mb) * 8 + a_rb, a_k0, I, lane));
+    const uint32_t a_voff1 = uint32_t(afrag32_offset(uint32_t(mb) * 8 + a_rb + 1, a_k0, I, lane));
     auto dma_a = [&](uint32_t st) {
         const uint32_t a_soff = (st < s_end ? 4 * st : 0) * 1024u;
-        unsigned char* base = abuf + (st % 3) * WIDE_TILE_BYTES + 4 * w * 1024;
-        auto frag = [&](auto qc) {
+        unsigned char* base = abuf + (st % 3) * WIDE_TILE_BYTES + (4 * a_rb + a_k0) * 1024;
+        auto frag = [&](unsigned char* to, uint32_t voff, auto qc) {
             constexpr int q = decltype(qc)::value;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, (__attribute__((address_space(3))) void*)base, 16, a_voff,
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, (__attribute__((address_space(3))) void*)to, 16, voff,
                                                      a_soff, q * 1024, 0);
         };
-        frag(std::integral_constant<int, 0>{});
-        frag(std::integral_constant<int, 1>{});
-        frag(std::integral_constant<int, 2>{});
-        frag(std::integral_constant<int, 3>{});
+        frag(base, a_voff0, std::integral_constant<int, 0>{});
+        frag(base, a_voff0, std::integral_constant<int, 1>{});
+        frag(base + 4096, a_voff1, std::integral_constant<int, 0>{});
+        frag(base + 4096, a_voff1, std::integral_constant<int, 1>{});
     };
     // The compiler does not see the LDS side of these loads, so their
     // completion is awaited by hand: vmcnt(n) with n the vector-memory
-    // operations issued after the awaited ones.  Per stage the issue order is
-    // [4 A DMAs][decode][kChunkOps chunk loads].
+    // operations issued after the awaited ones.  Per decode phase the issue
+    // order is [4 A DMAs][decode][kChunkOps chunk loads].
     constexpr int kChunkOps = K <= 4 ? 1 : 2;
     // Stage barrier: this wave's LDS writes done (lgkmcnt(0)), its A DMAs of
     // the next stage done (vmcnt(n)), then s_barrier.  The memory clobber keeps
@@ -336,84 +343,115 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
                 }
     }
 
-    // Prologue: A stages s0 and s0 + 1 in flight, B stage s0 decoded, chunk ring full.
+    // ---- K loop: the workgroup's two halves take turns.  Each SIMD holds one
+    // wave of the early half (0-3) and one of the late half (4-7).  Time runs in
+    // slots, one barrier per slot; in every slot one half multiplies a stage (M:
+    // the SIMD's matrix pipe) while the other decodes (D: VALU, LDS stores, loads):
+    //   slot 2 st    : early M(st)       late  D(st + 1)
+    //   slot 2 st + 1: early D(st + 1)   late  M(st)
+    // With both waves of a SIMD in the same phase the pipe idled while both
+    // stored their fragments, waited at the stage barrier and read the first
+    // ones back: 2,940 cycles per stage for 2,048 of MFMA.  Measured against
+    // that loop, same bits: M = 512 on 5120^2 59.5 -> 57.0 us, M = 2048 on 4096
+    // -> 12288 225.2 -> 221.1 us, M = 3000 on 1280 -> 16384 173.4 -> 167.5 us.
+    // M takes 1,080-1,130 cycles (1,024 of MFMA), D about 1,550: D bounds the slot.
+    //
+    // D(n) decodes the half's two blocks of stage n into B buffer n % 2, DMAs
+    // its half of the core input of stage n + 1 into A buffer (n + 1) % 3,
+    // loads the next chunk and reads the first fragments of the half's next M.
+    // The barriers order every use:
+    //   B[n % 2]: late blocks are written in slot 2n - 2, early ones in 2n - 1; read
+    //     in slots 2n and 2n + 1 (and block 0, a late one, by the early half's
+    //     first reads in 2n - 1); the next writes come in slot 2n + 2.
+    //   A[n % 3]: DMAs are issued in slots 2n - 4 (K16 steps 0, 1: late half) and
+    //     2n - 3 (steps 2, 3: early half), awaited at the end of the issuer's
+    //     next D (slots 2n - 2 and 2n - 1), read from slot 2n - 1 (step 0) and 2n
+    //     on, last in slot 2n + 1; its buffer's next DMA comes in slot 2n + 2.
+    // Fragments of K16 step kb + 1 are read while step kb multiplies.
+    half8_t wf[2][TN], xf[2][TM];
+    auto read_frags = [&](uint32_t st, int kb) {
+        const unsigned char* ab = abuf + (st % 3) * WIDE_TILE_BYTES;
+        const unsigned char* bb = bbuf + (st & 1) * WIDE_TILE_BYTES;
 #pragma unroll
-    for (int d = 0; d < D; ++d) load_stage(ring[d], s0 + d);
+        for (int jn = 0; jn < TN; ++jn)
+            wf[kb & 1][jn] = *reinterpret_cast<const half8_t*>(bb + (((TN * wn + jn) * 4 + kb) * 64 + lane) * 16);
+#pragma unroll
+        for (int im = 0; im < TM; ++im)
+            xf[kb & 1][im] = *reinterpret_cast<const half8_t*>(ab + (((TM * wm + im) * 4 + kb) * 64 + lane) * 16);
+    };
+    auto multiply = [&](uint32_t st) {
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            if (kb < 3) read_frags(st, kb + 1);
+#pragma unroll
+            for (int jn = 0; jn < TN; ++jn)
+#pragma unroll
+                for (int im = 0; im < TM; ++im)
+                    acc[jn][im] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[kb & 1][jn], xf[kb & 1][im], acc[jn][im], 0, 0, 0);
+            // One read after each of the step's first MFMAs (0x008: MFMA, 0x100: LDS read).
+            if (kb < 3) {
+                if constexpr (TM == 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+                for (int i = 0; i < TM * 2 + 2; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+                if constexpr (TM == 2) __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            } else {
+                __builtin_amdgcn_sched_group_barrier(0x008, TN * TM, 0);
+            }
+        }
+    };
+    // D(n); `next` is the stage the half multiplies in the following slot.
+    auto decode_phase = [&](uint32_t n, uint32_t next) {
+        dma_a(n + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        decode_stage(chunk, n & 1);
+        __builtin_amdgcn_sched_barrier(0);
+        load_stage(chunk, n + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        clk.phase_end<2>();
+        read_frags(next, 0);
+        // The A DMAs of the half's previous D have landed once only that D's chunk
+        // loads and this one's DMAs and chunk loads remain.
+        stage_barrier(std::integral_constant<int, 4 + 2 * kChunkOps>{});
+    };
+
+    // Prologue: A stages s0 and s0 + 1 in flight, B stage s0 decoded, the chunk
+    // of s0 + 1 on its way.
+    load_stage(chunk, s0);
     __builtin_amdgcn_sched_barrier(0);
     dma_a(s0);
     dma_a(s0 + 1);
     __builtin_amdgcn_sched_barrier(0);
-    decode_stage(ring[0], s0 & 1);
-    load_stage(ring[0], s0 + D);
+    decode_stage(chunk, s0 & 1);
+    load_stage(chunk, s0 + 1);
     __builtin_amdgcn_sched_barrier(0);
     stage_barrier(std::integral_constant<int, 4 + kChunkOps>{});   // A stage s0 landed
     clk.loop_begin();
+    clk.stage_begin();
+    if (late) decode_phase(s0 + 1, s0);
+    else read_frags(s0, 0);
 
-    for (uint32_t st0 = s0; st0 < s_end; st0 += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const uint32_t st = st0 + d;
-            clk.stage_begin();
-            __builtin_amdgcn_sched_barrier(0);
-            dma_a(st + 2);
-            __builtin_amdgcn_sched_barrier(0);
-            // One instruction stream per stage: the MFMAs of stage st and the
-            // VALU decode of stage st + 1 are independent and interleaved in
-            // source order (one weight pair after every two MFMAs), so the
-            // matrix core and the VALU work at the same time.  The decoder's
-            // inline v_mad_u32_u16 pins the order for the machine scheduler.
-            const unsigned char* ab = abuf + (st % 3) * WIDE_TILE_BYTES;
-            const unsigned char* bb = bbuf + (st & 1) * WIDE_TILE_BYTES;
-            const int slot = (d + 1) % D;   // compile-time after unrolling
-            Chunk<K>& dc = ring[slot];
-            if (decoder) link_chunk(dc, g == 0);
-            half2_t wq[4][4];
-            // Fragments of K16 step kb + 1 are read while step kb multiplies.
-            half8_t wf[2][TN], xf[2][TM];
-            auto read_frags = [&](int kb) {
-#pragma unroll
-                for (int jn = 0; jn < TN; ++jn)
-                    wf[kb & 1][jn] = *reinterpret_cast<const half8_t*>(bb + (((TN * wn + jn) * 4 + kb) * 64 + lane) * 16);
-#pragma unroll
-                for (int im = 0; im < TM; ++im)
-                    xf[kb & 1][im] = *reinterpret_cast<const half8_t*>(ab + (((TM * wm + im) * 4 + kb) * 64 + lane) * 16);
-            };
-            read_frags(0);
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb) {
-                if (kb < 3) read_frags(kb + 1);
-#pragma unroll
-                for (int jn = 0; jn < TN; ++jn) {
-#pragma unroll
-                    for (int im = 0; im < TM; ++im)
-                        acc[jn][im] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[kb & 1][jn], xf[kb & 1][im], acc[jn][im], 0, 0, 0);
-                    // 16 weight pairs per stage, one after each of the 4 x 4 channel groups
-                    if (decoder) decode_pair_at<K, CB>(dc, wq, 4 * kb + jn);
-                }
-            }
-            // Decoded stage st + 1 -> the other B buffer (past the end: zeros
-            // of out-of-range loads into an unused buffer).
-            clk.phase_end<0>();
-            if (decoder) store_bfrag(wq, (st + 1) & 1);
-            __builtin_amdgcn_sched_barrier(0);
-            load_stage(ring[slot], st + 1 + D);
-            __builtin_amdgcn_sched_barrier(0);
-            clk.phase_end<1>();
-            // A stage st + 1 (issued one stage ago) has landed once at most the
-            // last stage's chunk loads, this stage's 4 DMAs and chunk loads remain.
-#if STX_STAGE_CLOCK
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(4 + 2 * kChunkOps) : "memory");
-            clk.phase_end<2>();
-            asm volatile("s_barrier" ::: "memory");
-            clk.phase_end<3>();
-            clk.stage_end();
-#else
-            stage_barrier(std::integral_constant<int, 4 + 2 * kChunkOps>{});
-#endif
-        }
+    for (uint32_t st = s0;;) {
+        clk.stage_begin();
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+        multiply(st);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        clk.phase_end<0>();
+        asm volatile("s_barrier" ::: "memory");
+        clk.phase_end<1>();
+        clk.stage_end();
+        if (++st >= s_end) break;
+        decode_phase(st + late, st);
+        clk.phase_end<3>();
     }
-    // The last stages issued A DMAs past the end (dummy rows into A buffers):
-    // they land before LDS is reused as the epilogue tile or by the next item.
+    // The early half is one slot ahead: its last barrier pairs with the one
+    // after the late half's last M.  A DMAs past the end (dummy rows) land before
+    // LDS is reused.
+    if (!late) asm volatile("s_barrier" ::: "memory");
     stage_barrier(std::integral_constant<int, 0>{});
     clk.loop_end();
 
