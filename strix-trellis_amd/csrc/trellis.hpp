@@ -116,13 +116,11 @@ __device__ __forceinline__ void link_chunk(Chunk<K>& c, bool first_of_tile) {
 
 // ---------------------------------------------------------------------------
 // Window of the state at chunk position (V, F): fragment lane 4g+V, fragment F.
-// Its 16 bits end (8V+F+1)*K bits after the chunk start.  Returns a register
-// whose low (HI = false) or high (HI = true) 16 bits are the state; the other
-// half is don't-care, because every consumer reads 16-bit operands.  Two
-// windows 16 bits apart share one v_alignbit (K = 2, 4, 8).  Other widths have
-// no such pairs, so their windows take the high half only where it is a word's
-// own high half (no v_alignbit); a v_pk_* product of a high half counts as a
-// high-half write for the compiler, whose next reader then waits a state.
+// Its 16 bits end (8V+F+1)*K bits after the chunk start; state() returns them
+// zero-extended.  Two windows 16 bits apart share one v_alignbit (K = 1, 2, 4,
+// 8): the lower is its low half (v_and), the upper its high half (v_lshrrev).
+// Other widths have no such pairs: a window inside one word is one v_bfe, one
+// that crosses words a v_alignbit and a v_and.
 // ---------------------------------------------------------------------------
 template <int K, int V, int F>
 struct Window {
@@ -130,41 +128,33 @@ struct Window {
     static constexpr int shift = 32 * K - end;   // distance of the window LSB from the chunk LSB
     static constexpr int q = shift / 32;
     static constexpr int r = shift % 32;
-    static constexpr bool hi = r == 16 || (r > 16 && 16 % K == 0);
+    static constexpr bool paired = 16 % K == 0;
+    static constexpr bool hi = r == 16 || (r > 16 && paired);
     static constexpr int align = hi ? r - 16 : r;
 
-    __device__ __forceinline__ static uint32_t reg(const Chunk<K>& c) {
-        if constexpr (align == 0) {
-            return c.template lsb<q>();
-        } else {
-            return __builtin_amdgcn_alignbit(c.template lsb<q + 1>(), c.template lsb<q>(), align);
-        }
+    __device__ __forceinline__ static uint32_t state(const Chunk<K>& c) {
+        uint32_t w;
+        if constexpr (align == 0) w = c.template lsb<q>();
+        else if constexpr (!paired && r < 16) return (c.template lsb<q>() >> r) & 0xFFFFu;
+        else w = __builtin_amdgcn_alignbit(c.template lsb<q + 1>(), c.template lsb<q>(), align);
+        return hi ? w >> 16 : w & 0xFFFFu;
     }
 };
 
 // ---------------------------------------------------------------------------
-// Codebook products p = state * M (+ C) mod 2^32 on a 16-bit half-register
-// operand: p = lo16(s)*M_lo + ((lo16(s)*M_hi mod 2^16) << 16) (+ C).
-// v_pk_mul_lo_u16 with op_sel produces the shifted high product directly and
-// v_mad_u32_u16 ignores the upper half of its 16-bit operands.
+// Codebook products p = state * M (+ C) mod 2^32.  v_mul_lo_u32 issues at the
+// full VOP3 rate here (4.25 cycles per wave and SIMD with two or more waves,
+// measured; v_and and v_lshrrev, being VOP2, take 2.4), so a zero-extended
+// state and one multiply (6.7 cycles) beat the two-instruction product of a
+// half-register operand, v_pk_mul_lo_u16 for the high part and v_mad_u32_u16
+// (8.5), and need none of the wait states that follow a high-half operand.
+// The asm keeps the compiler, which prices v_mul_lo_u32 at quarter rate, from
+// splitting it.
 // ---------------------------------------------------------------------------
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-
-template <uint32_t M, bool HI>
-__device__ __forceinline__ uint32_t product16(uint32_t src) {
-    constexpr uint32_t mlo = M & 0xFFFFu;
-    const u16x2 sv = __builtin_bit_cast(u16x2, src);
-    const unsigned short s = HI ? sv.y : sv.x;
-    const u16x2 splat = {s, s};
-    const u16x2 mhi = {0, (unsigned short)(M >> 16)};
-    // (0, s*M_hi mod 2^16): the compiler selects v_pk_mul_lo_u16 with op_sel.
-    const uint32_t hs = __builtin_bit_cast(uint32_t, splat * mhi);
+template <uint32_t M>
+__device__ __forceinline__ uint32_t product32(uint32_t state) {
     uint32_t p;
-    if constexpr (!HI) {
-        asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(p) : "v"(src), "s"(mlo), "v"(hs));
-    } else {
-        asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(p) : "v"(src), "s"(mlo), "v"(hs));
-    }
+    asm("v_mul_lo_u32 %0, %1, %2" : "=v"(p) : "v"(state), "s"(M));
     return p;
 }
 
@@ -173,11 +163,11 @@ constexpr uint32_t MCG_M = 0xCBAC1FEDu;
 constexpr uint32_t INST3_M = 89226354u;
 constexpr uint32_t INST3_C = 64248484u;
 
-template <int CB, bool HI>
-__device__ __forceinline__ uint32_t codebook_product(uint32_t src) {
-    if constexpr (CB == CB_MUL1) return product16<MUL1_M, HI>(src);
-    else if constexpr (CB == CB_MCG) return product16<MCG_M, HI>(src);
-    else return product16<INST3_M, HI>(src) + INST3_C;
+template <int CB>
+__device__ __forceinline__ uint32_t codebook_product(uint32_t state) {
+    if constexpr (CB == CB_MUL1) return product32<MUL1_M>(state);
+    else if constexpr (CB == CB_MCG) return product32<MCG_M>(state);
+    else return product32<INST3_M>(state) + INST3_C;
 }
 
 // mul1: b = sum of the four bytes of p; value = RN16((1024+b)*h(0x1EEE) + h(0xC931))
@@ -205,8 +195,8 @@ template <int K, int CB, int V, int F>
 __device__ __forceinline__ half2_t decode_pair(const Chunk<K>& c) {
     using A = Window<K, V, F>;
     using B = Window<K, V, F + 1>;
-    const uint32_t pa = codebook_product<CB, A::hi>(A::reg(c));
-    const uint32_t pb = codebook_product<CB, B::hi>(B::reg(c));
+    const uint32_t pa = codebook_product<CB>(A::state(c));
+    const uint32_t pb = codebook_product<CB>(B::state(c));
     if constexpr (CB == CB_MUL1) {
         return mul1_pair(pa, pb);
     } else {
