@@ -457,32 +457,72 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
 
     // Lane l holds rows 32 (TM wm + im) + l % 32 of the tile and, per MFMA
     // tile jn and accumulator r, channel 32 jn + 8 (r / 4) + 4 (l / 32) + r % 4
-    // of the wave's group: four consecutive channels per (jn, r / 4), stored
-    // as one 16-byte access.  Row-major [rows][N] F32 outputs of the tile's 256
-    // rows go through a buffer resource sized to the rows below M, so accesses
-    // to rows >= M are dropped (stores) or read zeros (loads).
+    // of the wave's group: four consecutive channels per (jn, r / 4).  Stored
+    // from there, each 16-byte store instruction touches 32 rows with 32 bytes
+    // apiece, and the L2 takes those requests at a quarter of its line rate.  So
+    // each 32-row block of a wave turns around in the wave's own 16 KiB of LDS
+    // (row-major, 16-byte unit u of row r at unit u ^ r, free of bank conflicts both
+    // ways): afterwards lane l holds channels 4 (l % 32) .. + 3 of row 2 i +
+    // l / 32, and a store instruction writes two whole 512-byte row segments.
+    // A wave's LDS operations are in order, so no barrier is needed.  Measured:
+    // 22,200 -> 13,600 cycles per tile (plane stores 10,800 -> 8,700); calls, same
+    // bits, M = 512 on 5120^2 55.8 -> 54.7 us, M = 2048 on 4096 -> 12288 220 -> 212
+    // us, M = 3000 on 1280 -> 16384 166 -> 154 us.
     const uint32_t row0 = uint32_t(mb) * 256;
     const uint32_t slab_bytes = (a.M - row0 < 256u ? a.M - row0 : 256u) * N * 4u;
-    const uint32_t out_off = ((32u * TM * wm + (lane & 31)) * N + uint32_t(BN) * c + 128u * wn + 4u * (lane >> 5)) * 4u;
-    auto acc4 = [&](int jn, int im, int r4) {
-        return u32x4{bits_of(acc[jn][im][4 * r4]), bits_of(acc[jn][im][4 * r4 + 1]), bits_of(acc[jn][im][4 * r4 + 2]),
-                     bits_of(acc[jn][im][4 * r4 + 3])};
+    const uint32_t hl = uint32_t(lane) >> 5, l5 = uint32_t(lane) & 31u;
+    unsigned char* turn = smem + 16384 * w;
+    const uint32_t turn_w = l5 * 512u + ((hl ^ l5) * 16u), turn_r = hl * 512u + ((l5 ^ hl) * 16u);
+    auto turn_put = [&](const float (&v)[TN][16]) {
+#pragma unroll
+        for (int jn = 0; jn < TN; ++jn)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+                *reinterpret_cast<u32x4*>(turn + (turn_w ^ ((8 * jn + 2 * r4) * 16))) =
+                    u32x4{bits_of(v[jn][4 * r4]), bits_of(v[jn][4 * r4 + 1]), bits_of(v[jn][4 * r4 + 2]),
+                          bits_of(v[jn][4 * r4 + 3])};
     };
+    auto turn_get = [&](int i) {
+        return *reinterpret_cast<const float4_t*>(turn + (turn_r ^ (2 * i * 16)) + 1024 * i);
+    };
+    // Byte offset within the tile's rows of the lane's channels in row
+    // 32 (TM wm + im) + 2 i + l / 32.  Rows go through a buffer resource sized
+    // to the rows below M, so accesses to rows >= M are dropped (stores) or read
+    // zeros (loads); the whole offset is the vector one, which the range check
+    // covers.
+    const uint32_t out_off = ((32u * TM * wm + hl) * N + uint32_t(BN) * c + 128u * wn + 4u * l5) * 4u;
+    auto row_off = [&](int im, int i) { return out_off + uint32_t(32 * im + 2 * i) * (N * 4u); };
+    auto take = [&](auto imc, float (&v)[TN][16]) {
+        constexpr int im = decltype(imc)::value;
+#pragma unroll
+        for (int jn = 0; jn < TN; ++jn)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[jn][r] = acc[jn][im][r];
+    };
+    constexpr std::integral_constant<int, 0> first{};
+    constexpr std::integral_constant<int, TM - 1> last{};
+    float v[TN][16];
 
     if (!HANDOFF && a.splits > 1) {
         const auto prsrc = make_rsrc(a.planes + (uint64_t(split) * a.M + row0) * N, slab_bytes);
+        auto put_plane = [&](auto imc) {
+            take(imc, v);
+            turn_put(v);
 #pragma unroll
-        for (int im = 0; im < TM; ++im)
-#pragma unroll
-            for (int jn = 0; jn < TN; ++jn)
-#pragma unroll
-                for (int r4 = 0; r4 < 4; ++r4)
-                    __builtin_amdgcn_raw_buffer_store_b128(acc4(jn, im, r4), prsrc, out_off + (32 * jn + 8 * r4) * 4,
-                                                           32 * im * N * 4, 0);
+            for (int i = 0; i < 16; ++i)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, turn_get(i)), prsrc,
+                                                       row_off(decltype(imc)::value, i), 0, 0);
+        };
+        put_plane(first);
+        if constexpr (TM == 2) put_plane(last);
         clk.record(a, kind, t, s0);
         return;
     }
 
+    auto acc4 = [&](int jn, int im, int r4) {
+        return u32x4{bits_of(acc[jn][im][4 * r4]), bits_of(acc[jn][im][4 * r4 + 1]), bits_of(acc[jn][im][4 * r4 + 2]),
+                     bits_of(acc[jn][im][4 * r4 + 3])};
+    };
     if (HANDOFF && kind == kItemHead) {
 #pragma unroll
         for (int jn = 0; jn < TN; ++jn)
@@ -505,17 +545,14 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
     }
 
     // ---- Epilogue: H128 per row in registers, then the output stage ----
-    // The tile's svh (and bias) go to LDS by DMA while the butterflies run:
-    // wave 0 brings BN x 2 B of svh to bytes [0, 1024), wave 1 BN x 4 B of
-    // bias to [1024, 2048) (lanes past the end read zeros).
+    // The lane's output-stage operands (channels 4 (l % 32) .. + 3 after the
+    // turn) arrive while the butterflies run.  A missing bias reads through an
+    // empty range and adds -0.0 instead, which leaves every value (signed zeros
+    // included) unchanged.
     const bool has_bias = a.bias != nullptr;
-    if (w < (has_bias ? 2 : 1)) {
-        const void* src = w == 0 ? static_cast<const void*>(a.svh + uint64_t(BN) * c)
-                                 : static_cast<const void*>(a.bias + uint64_t(BN) * c);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(src, w == 0 ? BN * 2 : BN * 4),
-                                                 (__attribute__((address_space(3))) void*)(smem + 1024 * w), 16,
-                                                 uint32_t(lane) * 16u, 0, 0, 0);
-    }
+    const uint32_t lane_ch = uint32_t(BN) * c + 128u * wn + 4u * l5;
+    const u32x2 svq = ld_global(reinterpret_cast<const u32x2*>(a.svh + lane_ch));
+    const u32x4 bq = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(a.bias, has_bias ? N * 4u : 0u), lane_ch * 4u, 0, 0);
     // Butterfly levels in the reference's order, channel bit 0 first; lower
     // element a + b, upper element a - b.  Channel bits 0, 1, 3, 4 are bits of
     // r, bits 5, 6 of jn, bit 2 is lane bit 5.  The values of one row block
@@ -526,11 +563,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
         hi = x - y;
     };
     auto h128 = [&](auto imc, float (&v)[TN][16]) {
-        constexpr int im = decltype(imc)::value;
-#pragma unroll
-        for (int jn = 0; jn < TN; ++jn)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) v[jn][r] = acc[jn][im][r];
+        take(imc, v);
 #pragma unroll
         for (int jn = 0; jn < TN; ++jn) {
             float* t = v[jn];
@@ -573,59 +606,45 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
     };
 
     // Output stage per element, as output_value() with the operands in
-    // registers: RN32(h * svh), + bias, * alpha, + RN32(beta * y).  A missing
-    // bias adds -0.0, which leaves every value (signed zeros included)
-    // unchanged; y is read only when beta != 0.
-    const uint16_t* sv_lds = reinterpret_cast<const uint16_t*>(smem);
-    const float* bias_lds = reinterpret_cast<const float*>(smem + 1024);
-    const uint32_t lc0 = 128u * wn + 4u * (lane >> 5);   // first channel of the lane within the tile
+    // registers: RN32(h * svh), + bias, * alpha, + RN32(beta * y); y is read only
+    // when beta != 0.
+    const float sv[4] = {half_bits_to_float(uint16_t(svq.x & 0xFFFFu)), half_bits_to_float(uint16_t(svq.x >> 16)),
+                         half_bits_to_float(uint16_t(svq.y & 0xFFFFu)), half_bits_to_float(uint16_t(svq.y >> 16))};
+    const float bv[4] = {has_bias ? float_of(bq.x) : -0.0f, has_bias ? float_of(bq.y) : -0.0f,
+                         has_bias ? float_of(bq.z) : -0.0f, has_bias ? float_of(bq.w) : -0.0f};
     const auto yrsrc = make_rsrc(a.y + uint64_t(row0) * N, slab_bytes);
-    auto emit = [&](auto imc, const float (&v)[TN][16], auto with_beta) {
+    auto emit = [&](auto imc, auto with_beta) {
         constexpr int im = decltype(imc)::value;
         constexpr bool BETA = decltype(with_beta)::value;
 #pragma unroll
-        for (int jn = 0; jn < TN; ++jn)
+        for (int i = 0; i < 16; ++i) {
+            const uint32_t off = row_off(im, i);
+            const float4_t h = turn_get(i);
+            u32x4 old{};
+            if constexpr (BETA) old = __builtin_amdgcn_raw_buffer_load_b128(yrsrc, off, 0, 0);
+            u32x4 o;
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                const uint32_t lc = lc0 + 32 * jn + 8 * r4;
-                const uint2 sv = *reinterpret_cast<const uint2*>(sv_lds + lc);
-                const float4_t bv = has_bias ? *reinterpret_cast<const float4_t*>(bias_lds + lc)
-                                             : float4_t{-0.0f, -0.0f, -0.0f, -0.0f};
-                const uint32_t sw[4] = {sv.x & 0xFFFFu, sv.x >> 16, sv.y & 0xFFFFu, sv.y >> 16};
-                const uint32_t off = out_off + (32 * jn + 8 * r4) * 4;
-                u32x4 old{};
-                if constexpr (BETA) old = __builtin_amdgcn_raw_buffer_load_b128(yrsrc, off, 32 * im * N * 4, 0);
-                u32x4 o;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float y = rn32(v[jn][4 * r4 + e] * half_bits_to_float(uint16_t(sw[e])));
-                    y = rn32(y + bv[e]);
-                    y = rn32(y * a.alpha);
-                    if constexpr (BETA) y = rn32(y + rn32(a.beta * float_of(old[e])));
-                    o[e] = bits_of(y);
-                }
-                __builtin_amdgcn_raw_buffer_store_b128(o, yrsrc, off, 32 * im * N * 4, 0);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int e = 0; e < 4; ++e) {
+                float y = rn32(h[e] * sv[e]);
+                y = rn32(y + bv[e]);
+                y = rn32(y * a.alpha);
+                if constexpr (BETA) y = rn32(y + rn32(a.beta * float_of(old[e])));
+                o[e] = bits_of(y);
             }
+            __builtin_amdgcn_raw_buffer_store_b128(o, yrsrc, off, 0, 0);
+        }
     };
     // Row block by row block: each one's results are stored before the next
     // one's butterflies, which bounds the live values.
     const bool use_beta = a.beta != 0.0f;
-    auto emit_any = [&](auto imc, const float (&v)[TN][16]) {
-        if (use_beta) emit(imc, v, std::true_type{});
-        else emit(imc, v, std::false_type{});
+    auto finish = [&](auto imc) {
+        h128(imc, v);
+        turn_put(v);
+        if (use_beta) emit(imc, std::true_type{});
+        else emit(imc, std::false_type{});
     };
-    float v[TN][16];
-    constexpr std::integral_constant<int, 0> first{};
-    h128(first, v);
-    __builtin_amdgcn_s_waitcnt(0);   // this wave's svh / bias DMA landed
-    __syncthreads();
-    emit_any(first, v);
-    if constexpr (TM == 2) {
-        constexpr std::integral_constant<int, 1> second{};
-        h128(second, v);
-        emit_any(second, v);
-    }
+    finish(first);
+    if constexpr (TM == 2) finish(last);
     clk.record(a, kind, t, s0);
 }
 
