@@ -6,12 +6,13 @@
 namespace stx {
 
 // Input stage of RB rows x 128 channels into MFMA A-fragment order: RB = 16
-// for the 16x32 fragments of gemm_kernel, RB = 32 for the 32x16 fragments of
+// for the 16x32 fragments of gemm_narrow_kernel, RB = 32 for the 32x16 fragments of
 // gemm_wide_kernel.  Each wave stages RB / 4 rows (one 128-block each) into an
 // LDS tile; then every thread writes whole fragment lanes -- 8 consecutive
 // channels of one row, 16 contiguous bytes -- so each fragment (64 lanes x
 // 16 B) is one coalesced 1 KiB store.  Rows past M are zero.
-// Workgroup (0, 0) also clears the wide GEMM's `nflags` handoff flags.
+// Workgroup (0, 0) also clears the core's `nflags` flags: the wide one's handoff
+// flags or the narrow one's arrival counters.
 template <int RB>
 __global__ __launch_bounds__(256) void input_stage_frag_kernel(const float* x, const uint16_t* suh, uint32_t M,
                                                                uint32_t I, _Float16* afrag, uint32_t* flags,
@@ -56,19 +57,12 @@ __global__ __launch_bounds__(256) void input_stage_frag_kernel(const float* x, c
 }
 
 using GemmDispatch = hipError_t (*)(const GemmLaunch&);
-static const GemmDispatch gemm_table[8] = {gemm_dispatch<1>, gemm_dispatch<2>, gemm_dispatch<3>, gemm_dispatch<4>,
-                                           gemm_dispatch<5>, gemm_dispatch<6>, gemm_dispatch<7>, gemm_dispatch<8>};
+static const GemmDispatch gemm_narrow_table[8] = {
+    gemm_narrow_dispatch<1>, gemm_narrow_dispatch<2>, gemm_narrow_dispatch<3>, gemm_narrow_dispatch<4>,
+    gemm_narrow_dispatch<5>, gemm_narrow_dispatch<6>, gemm_narrow_dispatch<7>, gemm_narrow_dispatch<8>};
 static const GemmDispatch gemm_wide_table[8] = {gemm_wide_dispatch<1>, gemm_wide_dispatch<2>, gemm_wide_dispatch<3>,
                                                 gemm_wide_dispatch<4>, gemm_wide_dispatch<5>, gemm_wide_dispatch<6>,
                                                 gemm_wide_dispatch<7>, gemm_wide_dispatch<8>};
-
-// Row-block height: 256 halves the decode work per flop; 128 when the rows
-// would not fill a 256 block or when 256-row blocks leave most CUs idle.
-static uint32_t gemm_bm(uint64_t rows, uint32_t groups) {
-    if (rows <= 128) return 128;
-    const uint64_t wg256 = uint64_t(groups) * ((rows + 255) / 256);
-    return wg256 >= 256 ? 256 : 128;
-}
 
 #if STX_STAGE_CLOCK
 // Instrumented build only (build.py --stage-clock): where the wide kernel
@@ -86,8 +80,8 @@ hipError_t launch_gemm(const DeviceWeights& w, const LinearCall& call, hipStream
     _Float16* afrag = static_cast<_Float16*>(call.workspace);
     for (uint64_t r0 = 0; r0 < call.rows; r0 += pass) {
         const uint64_t m = call.rows - r0 < pass ? call.rows - r0 : pass;
-        // 256 x 256 tiles (32x16 fragments) once the rows fill them and N
-        // splits into 256-column blocks; 128-row tiles (16x32 fragments) otherwise.
+        // 256 x 256 tiles (32x16 fragments) once the rows fill them and N splits
+        // into 256-column blocks; the narrow core (16x32 fragments) otherwise.
         const bool wide = gemm_wide(m, w);
         const uint32_t rb = wide ? 32 : 16;
         const uint64_t mpad = (m + rb - 1) / rb * rb;
@@ -96,12 +90,15 @@ hipError_t launch_gemm(const DeviceWeights& w, const LinearCall& call, hipStream
         char* hbase = reinterpret_cast<char*>(call.workspace) + afrag_bytes(w, m);
         float* handoff = reinterpret_cast<float*>(hbase);
         uint32_t* flags = reinterpret_cast<uint32_t*>(hbase + align256(handoff_bytes(h.x)));
+        // Narrow pass: the arrival counters follow the planes.
+        uint32_t* counters = reinterpret_cast<uint32_t*>(
+            hbase + align256(uint64_t(wide ? 0 : narrow_splits(w)) * m * w.output * sizeof(float)));
         if (wide)
             hipLaunchKernelGGL(input_stage_frag_kernel<32>, dim3(w.input / 128, uint32_t(mpad / 32)), dim3(256), 0,
                                stream, x, w.suh, uint32_t(m), w.input, afrag, flags, h.x);
         else
             hipLaunchKernelGGL(input_stage_frag_kernel<16>, dim3(w.input / 128, uint32_t(mpad / 16)), dim3(256), 0,
-                               stream, x, w.suh, uint32_t(m), w.input, afrag, flags, 0u);
+                               stream, x, w.suh, uint32_t(m), w.input, afrag, counters, narrow_counters(m, w));
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         GemmLaunch l{};
@@ -127,10 +124,9 @@ hipError_t launch_gemm(const DeviceWeights& w, const LinearCall& call, hipStream
         l.args.clock = g_stage_clock;
 #endif
         l.codebook = w.codebook;
-        l.bm = gemm_bm(m, w.output / 128);
         l.stream = stream;
         auto fold_planes = [&]() -> hipError_t {
-            if (l.args.splits == 1) return hipSuccess;
+            if (!pass_folds(m, w)) return hipSuccess;
             LinearCall pc = call;
             pc.rows = m;
             pc.y = l.args.y;
@@ -138,7 +134,9 @@ hipError_t launch_gemm(const DeviceWeights& w, const LinearCall& call, hipStream
             return launch_plane_finish(w, pc, l.args.planes, l.args.splits, stream);
         };
         if (!wide) {
-            e = gemm_table[w.bits - 1](l);
+            l.bm = narrow_rows(m, w);
+            l.args.flags = counters;
+            e = gemm_narrow_table[w.bits - 1](l);
             if (e != hipSuccess) return e;
             e = fold_planes();
             if (e != hipSuccess) return e;

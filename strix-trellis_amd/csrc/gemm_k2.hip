@@ -1,8 +1,8 @@
-// Prefill GEMM kernels for K = 2 bits per weight (all codebooks): 128/256-row
-// blocks of 128 columns, and the 256 x 256 wide kernel.
+// Prefill GEMM kernels for K = 2 bits per weight (all codebooks): the narrow core
+// and the 256-row wide one.
 #include "gemm_wide.hpp"
 
 namespace stx {
-STX_INSTANTIATE_GEMM(2)
+STX_INSTANTIATE_GEMM_NARROW(2)
 STX_INSTANTIATE_GEMM_WIDE(2)
 }  // namespace stx

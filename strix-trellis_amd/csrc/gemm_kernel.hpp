@@ -1,30 +1,48 @@
 // Prefill GEMM on MFMA for gfx950: C[M][N] = A[M][I] . Q[I][N] with Q decoded
-// from the trellis on the fly, FP16 operands, FP32 accumulation, and the
-// output stage (H128 over N, svh, bias, alpha/beta) fused into the epilogue.
+// from the trellis on the fly, FP16 operands, FP32 accumulation.  This is the
+// narrow core: calls of fewer than 256 rows, and layers whose width is not a
+// multiple of 256 (reference src/wmma_tiled.hip:87-269, src/gemm.hip:15-76);
+// the rest run the wide core (gemm_wide.hpp).
 //
-// Replaces the reference's WMMA prefill cores (src/wmma_tiled.hip:87-269,
-// src/gemm.hip:15-76) with a CDNA4 design built around v_mfma_f32_16x16x32_f16:
+// Bound: the trellis decode (VALU) and, with few rows, latency.  K splits in
+// narrow_splits parts (a function of the layer only); a workgroup of four waves
+// owns 64 output columns and 16 TM rows of one part, small enough (32 KiB of
+// LDS) for two to five workgroups per CU, so that one's decode covers another's
+// barrier and loads.  Per stage of 128 channels:
+//   * every lane decodes one chunk: wave w the two input blocks of K32 step w,
+//     lanes 0-31 block 2w, lanes 32-63 block 2w + 1 (8 lanes per 16-column tile,
+//     four tiles), and stores its column fragments in MFMA B-operand order in
+//     LDS (double-buffered);
+//   * the four waves multiply as WM x (4 / WM): TM / WM row tiles by WM column
+//     tiles each, B fragments from LDS, A fragments from global memory (the L1
+//     serves the waves that share them) one stage ahead, in MFMA A-operand
+//     order, which the input-stage kernel wrote: one coalesced 16-byte load per
+//     lane and fragment.  WM balances the two sources: more waves along M read
+//     fewer A fragments twice and more B ones;
+//   * raw core rows go to planes[split][M][N] whatever the split count; with row
+//     blocks of 16 or 32 the last workgroup of a 128-column group folds them and
+//     applies the output stage itself, otherwise a second launch does
+//     (plane_finish_kernel).
+// Per-output accumulation: MFMA K32 steps in ascending K from +0 (the order
+// inside one MFMA step is the hardware's), then the planes in ascending split
+// order from +0; so a row has the same bits in every such call.
 //
-//   * workgroup tile BM x 128: 128 columns are one H128 output group, so the
-//     workgroup owns complete output rows of its group and applies the output
-//     stage itself; BM = 256 (8 waves as 4 x 2) or 128 (4 waves as 2 x 2);
-//     each wave computes a 64 x 64 block (4 x 4 MFMA tiles of 16 x 16);
-//   * K advances in stages of 128 channels (8 input blocks of 16).  In every
-//     stage the workgroup decodes 8 x 8 trellis tiles: a wave decodes 8/NW
-//     input blocks with the GEMV chunk decoder (lane = chunk g of tile jt) and
-//     stores each lane's four 8-deep column fragments straight into the MFMA
-//     B-operand order in LDS (double-buffered, 32 KiB per stage);
-//   * A is read from global memory (L2-resident: every column group re-reads
-//     it) in MFMA A-operand order, which the input-stage kernel already wrote:
-//     one fully coalesced 16-byte load per lane per 16 x 32 fragment;
-//   * per-output accumulation: MFMA K32 steps in ascending K from +0 (the
-//     order inside one MFMA step is the hardware's).
+// Measured against 128 x 128 and 256 x 128 tiles of the same order (64 KiB of
+// LDS, two waves along each dimension; 320 workgroups on 5120^2 that multiplied
+// 128 rows whatever M was), calls, same bits: 5120^2 K5 M = 16 / 24 / 64 / 128 /
+// 200 24.5 / 24.6 / 27.6 / 30.9 / 40.7 -> 14.2 / 16.6 / 21.6 / 25.6 / 32.8 us, 4096
+// -> 12288 K6 29.1 / 29.4 / 32.0 / 35.7 / 49.7 -> 17.9 / 20.7 / 24.4 / 31.9 / 43.5 us,
+// 1152 -> 5120 K4 M = 16 / 128 25.0 / 30.3 -> 11.8 / 16.4 us; 5120 -> 1152 K4 M =
+// 512 / 4096 31.5 / 143.9 -> 27.0 / 127.9 us.
 //
 // MFMA 16x16x32 f16 operand layout (lane l, e = 0..7 / 0..3):
 //   A: A[l % 16][8 (l / 16) + e]      B: B[8 (l / 16) + e][l % 16]
 //   D: D[4 (l / 16) + e][l % 16]
 #pragma once
+#include <type_traits>
+
 #include "backend.hpp"
+#include "gemv_kernel.hpp"
 #include "stages.hpp"
 
 namespace stx {
@@ -48,12 +66,12 @@ struct GemmArgs {
     // of K between a head and a tail workgroup, 256 q whole tiles.
     uint32_t q, x;
     float* handoff;           // [x][8 waves][128 accumulators][64 lanes]
-    uint32_t* flags;          // [x], 0 at launch
+    uint32_t* flags;          // [x], 0 at launch; narrow kernel: arrivals per 128-column group and row block
     uint32_t poll_limit;      // tail's polls before it takes a tile over
     // K split: `splits` workgroups per tile (narrow kernel: grid z, I/splits
     // channels each; wide kernel: grid y, stage ranges) write their raw core
-    // rows to planes[s][M][N], which a second launch folds in ascending s from
-    // +0 before the output stage.
+    // rows to planes[s][M][N], folded in ascending s from +0 before the output
+    // stage.
     uint32_t splits;
     float* planes;
 #if STX_STAGE_CLOCK
@@ -68,122 +86,106 @@ __host__ __device__ __forceinline__ uint64_t afrag_offset(uint32_t rb, uint32_t 
     return ((uint64_t(rb) * (I / 32) + kb) * 64 + lane) * 16;
 }
 
-constexpr int GEMM_STAGE_BLOCKS = 8;                              // input blocks per K stage
-constexpr int GEMM_BSTAGE_BYTES = 8 * 4 * 64 * 16;                // 8 tiles x 4 K32 x 64 lanes x 16 B
+constexpr int NARROW_BSTAGE_BYTES = 4 * 4 * 64 * 16;   // 4 tiles x 4 K32 steps x 64 lanes x 16 B
 
-template <int K, int CB, int BM>
-__global__ __launch_bounds__(2 * BM) void gemm_kernel(GemmArgs a) {
-    constexpr int WM = BM / 64, NW = 2 * WM, BPW = GEMM_STAGE_BLOCKS / NW;
-    extern __shared__ __align__(16) unsigned char smem[];   // 2 B stages; reused by the epilogue
+template <int K, int CB, int TM, bool FOLD>
+__global__ __launch_bounds__(256) void gemm_narrow_kernel(const uint32_t* trellis, const _Float16* afrag, uint32_t input,
+                                                         uint32_t output, uint32_t splits, uint32_t rows,
+                                                         GemmArgs args) {
+    // What the first loads need comes as scalar arguments, preloaded into SGPRs.
+    GemmArgs a = args;
+    a.trellis = trellis;
+    a.afrag = afrag;
+    a.I = input;
+    a.N = output;
+    a.splits = splits;
+    a.M = rows;
+    a.afrag_bytes = uint64_t((rows + 15) / 16 * 16) * input * 2;
+    constexpr int WM = TM >= 8 ? 4 : TM >= 2 ? 2 : 1, WN = 4 / WM;   // waves along M and N
+    constexpr int RT = TM / WM, CT = 4 / WN;              // row and column tiles per wave
+    constexpr int D = 3;                                  // chunk ring: stages in flight
+    __shared__ __align__(16) unsigned char smem[2 * NARROW_BSTAGE_BYTES];
     const int c = blockIdx.x, mb = blockIdx.y, split = blockIdx.z;
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int wm = w >> 1, wn = w & 1;
-    const int jt = lane >> 3, g = lane & 7;
-    // This workgroup's K range: stages (128 channels each) [split * stages, +stages).
+    const int wm = w / WN, wn = w % WN;
+    const int jt = (lane >> 3) & 3, g = lane & 7, odd = lane >> 5;
     const uint32_t I = a.I, N = a.N, stages = I / 128 / a.splits, kb0 = uint32_t(split) * stages * 4;
 
     constexpr uint32_t tile_bytes = 32u * K;
     const uint32_t row_bytes = (N >> 4) * tile_bytes;
     const auto wrsrc = make_rsrc(reinterpret_cast<const char*>(a.trellis) +
-                                     uint64_t(split) * stages * GEMM_STAGE_BLOCKS * row_bytes,
-                                 uint32_t(uint64_t(stages) * GEMM_STAGE_BLOCKS * row_bytes));
+                                     uint64_t(split) * stages * 8 * row_bytes,
+                                 uint32_t(uint64_t(stages) * 8 * row_bytes));
     const auto arsrc = make_rsrc(a.afrag, uint32_t(a.afrag_bytes));
-    const uint32_t lane_off = (8u * c + jt) * tile_bytes + g * 4u * K;
-
-    // Decode role: wave w decodes input blocks w*BPW .. w*BPW+BPW-1 of each
-    // stage.  Their chunks stream through a register ring D stages deep, so a
-    // chunk load has D stages of MFMA work to arrive from HBM.
-    constexpr int D = BPW == 1 ? 4 : 2;
-    Chunk<K> ring[D][BPW];
-    auto load_stage = [&](Chunk<K> (&dst)[BPW], uint32_t st) {
-#pragma unroll
-        for (int i = 0; i < BPW; ++i) {
-            const uint32_t blk = st * GEMM_STAGE_BLOCKS + w * BPW + i;
-            load_chunk(dst[i], wrsrc, st < stages ? blk * row_bytes + lane_off : 0x80000000u);
-        }
+    // The lane's chunk of stage st: tile 4c + jt of block 8 st + 2w + odd.
+    const uint32_t lane_off = uint32_t(2 * w + odd) * row_bytes + (4u * c + jt) * tile_bytes + g * 4u * K;
+    auto load_stage = [&](Chunk<K>& dst, uint32_t st) {
+        const bool live = st < stages;
+        load_chunk(dst, wrsrc, lane_off + (live ? 0u : 0x80000000u), live ? st * 8u * row_bytes : 0u);
     };
-    auto decode_stage = [&](Chunk<K> (&src)[BPW], int buf) {
-        unsigned char* base = smem + buf * GEMM_BSTAGE_BYTES;
-#pragma unroll
-        for (int i = 0; i < BPW; ++i) {
-            link_chunk(src[i], g == 0);
-            half2_t wq[4][4];
-            decode_chunk<K, CB>(src[i], wq);
-            const int kb = w * BPW + i;            // block within the stage
-            const int k32 = kb >> 1, kg = (kb & 1) * 2;
-            // fragment (column n, k-group) -> [tile][k32][lane = 16 * kgroup + n]
-            auto frag = [&](int n, int kgroup) -> uint32_t* {
-                return reinterpret_cast<uint32_t*>(base + ((jt * 4 + k32) * 64 + kgroup * 16 + n) * 16);
-            };
-            u32x4 f;
-            f = {as_u32(wq[0][0]), as_u32(wq[1][0]), as_u32(wq[2][0]), as_u32(wq[3][0])};
-            *reinterpret_cast<u32x4*>(frag(g, kg)) = f;
-            f = {as_u32(wq[0][1]), as_u32(wq[1][1]), as_u32(wq[2][1]), as_u32(wq[3][1])};
-            *reinterpret_cast<u32x4*>(frag(g, kg + 1)) = f;
-            f = {as_u32(wq[0][2]), as_u32(wq[1][2]), as_u32(wq[2][2]), as_u32(wq[3][2])};
-            *reinterpret_cast<u32x4*>(frag(g + 8, kg)) = f;
-            f = {as_u32(wq[0][3]), as_u32(wq[1][3]), as_u32(wq[2][3]), as_u32(wq[3][3])};
-            *reinterpret_cast<u32x4*>(frag(g + 8, kg + 1)) = f;
-        }
+    // Fragment (column n, k-group) of (tile, K32 step) -> lane 16 * kgroup + n.
+    const uint32_t wr = ((jt * 4 + w) * 64 + 32 * odd + g) * 16;
+    auto decode_stage = [&](Chunk<K>& src, uint32_t buf) {
+        unsigned char* base = smem + buf * NARROW_BSTAGE_BYTES + wr;
+        link_chunk(src, g == 0);
+        auto frag = [&](auto fc, int l) {
+            constexpr int F = decltype(fc)::value;
+            const uint32_t f0 = as_u32(decode_pair<K, CB, 0, F>(src)), f1 = as_u32(decode_pair<K, CB, 1, F>(src));
+            const uint32_t f2 = as_u32(decode_pair<K, CB, 2, F>(src)), f3 = as_u32(decode_pair<K, CB, 3, F>(src));
+            *reinterpret_cast<u32x4*>(base + l * 16) = u32x4{f0, f1, f2, f3};
+        };
+        frag(std::integral_constant<int, 0>{}, 0);    // rows 0-7 of column g
+        frag(std::integral_constant<int, 2>{}, 16);   // rows 8-15
+        frag(std::integral_constant<int, 4>{}, 8);    // rows 0-7 of column g + 8
+        frag(std::integral_constant<int, 6>{}, 24);   // rows 8-15
     };
 
-    // MFMA role: rows [mb*BM + 64 wm, +64), columns [64 wn, +64) of the group.
-    const uint32_t rb0 = (uint32_t(mb) * BM + 64 * wm) / 16;
-    auto load_a = [&](half8_t (&af)[4], uint32_t kb32) {
+    // A fragments of the wave's row tiles: slot k32 holds K32 step k32 of the
+    // current stage and is refilled with that step of the next stage once
+    // consumed.  Row tiles past the padded rows read out of range (zeros).
+    const uint32_t rb0 = uint32_t(mb) * TM + uint32_t(wm);
+    half8_t af[4][RT];
+    auto load_a = [&](half8_t (&dst)[RT], uint32_t kb32) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(
-                arsrc, uint32_t(afrag_offset(rb0 + i, kb0 + kb32, I, lane)), 0, 0);
-            af[i] = __builtin_bit_cast(half8_t, v);
-        }
+        for (int i = 0; i < RT; ++i)
+            dst[i] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                     arsrc, uint32_t(afrag_offset(rb0 + WM * i, kb0 + kb32, I, lane)), 0, 0));
     };
-    float4_t acc[4][4];
+    float4_t acc[RT][CT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < CT; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
+    Chunk<K> ring[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) load_stage(ring[d], d);
+#pragma unroll
+    for (int k32 = 0; k32 < 4; ++k32) load_a(af[k32], k32);
     decode_stage(ring[0], 0);
     load_stage(ring[0], D);
     __syncthreads();
 
-    // A ring: slot k32 holds the wave's four 16 x 32 fragments of K32 step
-    // k32 of the current stage and is refilled with the same step of the next
-    // stage as soon as it is consumed, so every A load has a full stage
-    // (16 MFMAs x 4 steps) to arrive from L2 / MALL.
-    half8_t af[4][4];
-#pragma unroll
-    for (int k32 = 0; k32 < 4; ++k32) load_a(af[k32], k32);
-    // Stage st's chunks sit in ring slot st % D; the loop is unrolled by D so
-    // slots are compile-time.  Loads stay unconditional (past the end they are
-    // out of range or repeat a valid A step); only the MFMAs are guarded.
     for (uint32_t st0 = 0; st0 < stages; st0 += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             const uint32_t st = st0 + d;
-            const bool live = st < stages;
-            const unsigned char* bbase = smem + (st & 1) * GEMM_BSTAGE_BYTES;
+            if (st >= stages) break;
+            const unsigned char* bbase = smem + (st & 1) * NARROW_BSTAGE_BYTES;
 #pragma unroll
             for (int k32 = 0; k32 < 4; ++k32) {
-                if (live) {
-                    half8_t bf[4];
+                half8_t bf[CT];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        bf[j] = *reinterpret_cast<const half8_t*>(bbase + (((4 * wn + j) * 4 + k32) * 64 + lane) * 16);
+                for (int j = 0; j < CT; ++j)
+                    bf[j] = *reinterpret_cast<const half8_t*>(bbase + (((CT * wn + j) * 4 + k32) * 64 + lane) * 16);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < RT; ++i)
 #pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[k32][i], bf[j], acc[i][j], 0, 0, 0);
-                }
-                const uint32_t next = (st + 1) * 4 + k32;
-                load_a(af[k32], next < stages * 4 ? next : k32);
+                    for (int j = 0; j < CT; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[k32][i], bf[j], acc[i][j], 0, 0, 0);
+                if (st + 1 < stages) load_a(af[k32], (st + 1) * 4 + k32);
             }
-            // Decode stage st + 1 into the other buffer while MFMAs drain, and
-            // refill its ring slot with stage st + 1 + D.  Past the end this
-            // decodes the zeros of out-of-range loads into an unused buffer.
+            if (st + 1 >= stages) break;
             const int slot = (d + 1) % D;   // compile-time after unrolling
             decode_stage(ring[slot], (st + 1) & 1);
             load_stage(ring[slot], st + 1 + D);
@@ -191,83 +193,121 @@ __global__ __launch_bounds__(2 * BM) void gemm_kernel(GemmArgs a) {
         }
     }
 
-    if (a.splits > 1) {
-        // Raw core rows of this split -> its plane (folded by a second launch).
-        float* plane = a.planes + uint64_t(split) * a.M * N;
+    float* plane = a.planes + uint64_t(split) * a.M * N + 64 * c + 16 * CT * wn + (lane & 15);
+    auto put_plane = [&](auto coherent) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < RT; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const uint32_t row = uint32_t(mb) * BM + 64 * wm + 16 * i + 4 * (lane >> 4) + e;
+                const uint32_t row = 16 * (rb0 + WM * i) + 4 * (lane >> 4) + e;
                 if (row < a.M) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) plane[uint64_t(row) * N + 128 * c + 64 * wn + 16 * j + (lane & 15)] = acc[i][j][e];
+                    for (int j = 0; j < CT; ++j) {
+                        float* to = plane + uint64_t(row) * N + 16 * j;
+                        if constexpr (decltype(coherent)::value) store_coherent(to, acc[i][j][e]);
+                        else *to = acc[i][j][e];
+                    }
                 }
             }
+    };
+    if constexpr (!FOLD) {
+        put_plane(std::false_type{});
         return;
-    }
-
-    // Epilogue, 64 rows (one wm) at a time through a [64][128] FP32 LDS tile.
-    float* tile = reinterpret_cast<float*>(smem);
-    for (int p = 0; p < WM; ++p) {
-        if (wm == p) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int row = 16 * i + 4 * (lane >> 4) + e;
-                        const int col = 64 * wn + 16 * j + (lane & 15);
-                        tile[row * 129 + col] = acc[i][j][e];
-                    }
-        }
+    } else {
+        put_plane(std::true_type{});
+        // The last of the column group's 2 S workgroups (two halves of 128
+        // columns) folds the planes.  The partials are agent-scope stores,
+        // complete (waited for, then a barrier) before the arrival; the last
+        // arrival reads them with device-coherent loads issued after the counter
+        // result, behind a barrier.
+        __builtin_amdgcn_s_waitcnt(0);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __syncthreads();
-        for (int rr = w; rr < 64; rr += NW) {
-            const uint32_t row = uint32_t(mb) * BM + 64 * p + rr;
-            float z0 = tile[rr * 129 + lane], z1 = tile[rr * 129 + lane + 64];
-            h32_wave(z0, z1);
-            if (row < a.M) {
-                const uint32_t n0 = 128 * c + lane, n1 = n0 + 64;
-                float* yr = a.y + uint64_t(row) * N;
-                const float o0 = output_element(z0, ld_global(a.svh + n0), a.bias, n0, a.alpha, a.beta, yr + n0);
-                const float o1 = output_element(z1, ld_global(a.svh + n1), a.bias, n1, a.alpha, a.beta, yr + n1);
-                yr[n0] = o0;
-                yr[n1] = o1;
+        int* last = reinterpret_cast<int*>(smem);
+        const uint32_t cg = uint32_t(c) >> 1;
+        if (tid == 0)
+            *last = __hip_atomic_fetch_add(a.flags + uint64_t(mb) * (N / 128) + cg, 1u, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT) == 2 * a.splits - 1;
+        __syncthreads();
+        if (!*last) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        // Wave w folds rows w, w + 4, ... of the block, P at a time, lane l
+        // columns 2l and 2l + 1: each plane from +0 in ascending split order, then
+        // H32 and the output stage (the order and operations of plane_finish_kernel).
+        constexpr int P = 4, SB = 8;
+        const uint32_t n0 = 128u * cg + 2u * uint32_t(lane);
+        const uint32_t svp = ld_global(reinterpret_cast<const uint32_t*>(a.svh + n0));
+        const bool has_bias = a.bias != nullptr;
+        const auto rb = make_rsrc(a.bias, has_bias ? N * 4u : 0u);
+        const gemv_f2_t bias = __builtin_bit_cast(gemv_f2_t, __builtin_amdgcn_raw_buffer_load_b64(rb, n0 * 4u, 0, 0));
+        const uint32_t end = (uint32_t(mb) + 1) * (16 * TM) < a.M ? (uint32_t(mb) + 1) * (16 * TM) : a.M;
+        for (uint32_t r0 = uint32_t(mb) * (16 * TM) + uint32_t(w); r0 < end; r0 += 4 * P) {
+            gemv_f2_t z[P];
+#pragma unroll
+            for (int i = 0; i < P; ++i) z[i] = gemv_f2_t{0.0f, 0.0f};
+            for (uint32_t s0 = 0; s0 < a.splits; s0 += SB) {
+                gemv_f2_t v[SB][P];
+#pragma unroll
+                for (int u = 0; u < SB; ++u)
+#pragma unroll
+                    for (int i = 0; i < P; ++i) {
+                        // Past the last split or row: a valid address again, unused.
+                        const uint32_t ss = s0 + u < a.splits ? s0 + u : s0;
+                        const uint32_t r = r0 + 4 * i < end ? r0 + 4 * i : r0;
+                        const auto ps = make_rsrc(a.planes + (uint64_t(ss) * a.M + r) * N, N * 4u);
+                        v[u][i] = poll_pair(ps, n0 * 4u, 0);
+                    }
+#pragma unroll
+                for (int u = 0; u < SB; ++u)
+                    if (s0 + u < a.splits)
+#pragma unroll
+                        for (int i = 0; i < P; ++i) {
+                            z[i].x = z[i].x + v[u][i].x;
+                            z[i].y = z[i].y + v[u][i].y;
+                        }
+            }
+            h32_pairs<P>(z);
+#pragma unroll
+            for (int i = 0; i < P; ++i) {
+                if (r0 + 4 * i >= end) break;
+                float* yr = a.y + uint64_t(r0 + 4 * i) * N + n0;
+                gemv_f2_t o;
+                o.x = output_value(z[i].x, uint16_t(svp), has_bias, bias.x, a.alpha, a.beta, yr);
+                o.y = output_value(z[i].y, uint16_t(svp >> 16), has_bias, bias.y, a.alpha, a.beta, yr + 1);
+                *(__attribute__((address_space(1))) gemv_f2_t*)(yr) = o;
             }
         }
-        __syncthreads();
     }
 }
 
 struct GemmLaunch {
     GemmArgs args;
     uint32_t codebook;
-    uint32_t bm;
+    uint32_t bm;              // narrow kernel: rows per workgroup (16, 32, 64, 128 or 256)
     uint32_t bn, col_blocks;  // wide kernel: tile width and column blocks launched
     hipStream_t stream;
 };
 
 template <int K>
-hipError_t gemm_dispatch(const GemmLaunch& l);
+hipError_t gemm_narrow_dispatch(const GemmLaunch& l);
 
-inline size_t gemm_lds_bytes(int bm) {
-    const size_t stages = 2 * size_t(GEMM_BSTAGE_BYTES);
-    const size_t epilogue = size_t(64) * 129 * 4;
-    (void)bm;
-    return stages > epilogue ? stages : epilogue;
-}
-
-#define STX_INSTANTIATE_GEMM(K)                                                                         \
-    template <>                                                                                         \
-    hipError_t gemm_dispatch<K>(const GemmLaunch& l) {                                                  \
-        using Fn = void (*)(GemmArgs);                                                                  \
-        static const Fn t256[3] = {gemm_kernel<K, 0, 256>, gemm_kernel<K, 1, 256>, gemm_kernel<K, 2, 256>}; \
-        static const Fn t128[3] = {gemm_kernel<K, 0, 128>, gemm_kernel<K, 1, 128>, gemm_kernel<K, 2, 128>}; \
-        const Fn fn = l.bm == 256 ? t256[l.codebook] : t128[l.codebook];                               \
-        const dim3 grid(l.args.N / 128, (l.args.M + l.bm - 1) / l.bm, l.args.splits);                   \
-        hipLaunchKernelGGL(fn, grid, dim3(2 * l.bm), gemm_lds_bytes(l.bm), l.stream, l.args);          \
-        return hipGetLastError();                                                                       \
+// Row tiles of 16 per workgroup: 1, 2 or 4 with the fold, 8 or 16 without.
+#define STX_INSTANTIATE_GEMM_NARROW(K)                                                                          \
+    template <>                                                                                                \
+    hipError_t gemm_narrow_dispatch<K>(const GemmLaunch& l) {                                                   \
+        using Fn = void (*)(const uint32_t*, const _Float16*, uint32_t, uint32_t, uint32_t, uint32_t, GemmArgs); \
+        static const Fn table[5][3] = {                                                                        \
+            {gemm_narrow_kernel<K, 0, 1, true>, gemm_narrow_kernel<K, 1, 1, true>, gemm_narrow_kernel<K, 2, 1, true>}, \
+            {gemm_narrow_kernel<K, 0, 2, true>, gemm_narrow_kernel<K, 1, 2, true>, gemm_narrow_kernel<K, 2, 2, true>}, \
+            {gemm_narrow_kernel<K, 0, 4, false>, gemm_narrow_kernel<K, 1, 4, false>, gemm_narrow_kernel<K, 2, 4, false>}, \
+            {gemm_narrow_kernel<K, 0, 8, false>, gemm_narrow_kernel<K, 1, 8, false>, gemm_narrow_kernel<K, 2, 8, false>}, \
+            {gemm_narrow_kernel<K, 0, 16, false>, gemm_narrow_kernel<K, 1, 16, false>, gemm_narrow_kernel<K, 2, 16, false>}}; \
+        const int ti = l.bm == 16 ? 0 : l.bm == 32 ? 1 : l.bm == 64 ? 2 : l.bm == 128 ? 3 : 4;                  \
+        const dim3 grid(l.args.N / 64, (l.args.M + l.bm - 1) / l.bm, l.args.splits);                           \
+        const GemmArgs& a = l.args;                                                                            \
+        hipLaunchKernelGGL(table[ti][l.codebook], grid, dim3(256), 0, l.stream, a.trellis, a.afrag, a.I, a.N,   \
+                           a.splits, a.M, a);                                                                  \
+        return hipGetLastError();                                                                              \
     }
 
 }  // namespace stx

@@ -152,8 +152,8 @@ uint32_t wide_splits(uint64_t m, const DeviceWeights& w) {
     return s > 1 ? uint32_t(s) : 1;
 }
 
-// K-split of the narrow (M < 256) kernel: N/128 column groups alone leave
-// most CUs idle (96 workgroups on 4096 -> 12288, 40 on 5120^2), so the input
+// K-split of the narrow kernel: N/128 column groups alone leave most CUs idle
+// (96 on 4096 -> 12288, 40 on 5120^2), so the input
 // splits in S power-of-two parts until the column groups x S reach the 256
 // CUs (S <= 16, whole 128-channel stages per split).  S depends on the layer
 // only, so every row of every M < 256 call has the same bits; it is part of
@@ -164,6 +164,30 @@ uint32_t narrow_splits(const DeviceWeights& w) {
     uint32_t s = 1;
     while (groups * s < 256 && s < 16 && stages % (2 * s) == 0) s *= 2;
     return s;
+}
+
+// Rows per workgroup of the narrow core: the fewest that hold the pass, so that
+// no row tile multiplies padding, up to 128; 256 halves the decode per row, but
+// only two such workgroups fit a CU, so it is taken where they fill the 256 CUs
+// at that (measured at 200 rows, 128 -> 256: 4096 -> 12288 46.2 -> 43.5, 1280 ->
+// 32768 42.3 -> 37.8, 5120^2 32.4 -> 32.8, 5120 -> 1152 20.7 -> 22.0 us).
+uint32_t narrow_rows(uint64_t m, const DeviceWeights& w) {
+    if (m <= 128) return m <= 16 ? 16 : m <= 32 ? 32 : m <= 64 ? 64 : 128;
+    return uint64_t(w.output / 64) * narrow_splits(w) * ((m + 255) / 256) >= 512 ? 256 : 128;
+}
+
+// Arrival counters (one per 128-column group and row block) of a narrow pass
+// whose workgroups fold the planes themselves, else 0.  The last arrival folds
+// a row block alone, which beats a launch of its own for up to 32 rows (5120^2
+// K5 M = 16 / 32: 17.0 / 18.3 -> 14.2 / 16.8 us) and loses from 64 on (22.2 -> 24.5).
+uint32_t narrow_counters(uint64_t m, const DeviceWeights& w) {
+    const uint32_t r = narrow_rows(m, w);
+    return !gemm_wide(m, w) && r <= 32 ? uint32_t((m + r - 1) / r) * (w.output / 128) : 0;
+}
+
+// Whether a launch of its own folds the pass's planes.
+bool pass_folds(uint64_t m, const DeviceWeights& w) {
+    return gemm_wide(m, w) ? wide_splits(m, w) > 1 : narrow_counters(m, w) == 0;
 }
 
 // K-split handoff of a wide pass with only 256 x 256 tiles: T = 256 q + x
@@ -184,12 +208,12 @@ Handoff gemm_handoff(uint64_t m, const DeviceWeights& w) {
 uint64_t handoff_bytes(uint32_t x) { return uint64_t(x) * 8 * 128 * 64 * sizeof(float); }
 
 // Workspace of one pass of m rows: fragment-order input, then the handoff's
-// partial accumulators and flags (wide) or the split planes (narrow).
+// partial accumulators and flags (wide) or the planes and the arrival counters
+// (narrow).
 uint64_t pass_workspace(const DeviceWeights& w, uint64_t m) {
-    if (!gemm_wide(m, w)) {
-        const uint32_t s = narrow_splits(w);
-        return afrag_bytes(w, m) + (s > 1 ? align256(uint64_t(s) * m * w.output * sizeof(float)) : 0);
-    }
+    if (!gemm_wide(m, w))
+        return afrag_bytes(w, m) + align256(uint64_t(narrow_splits(w)) * m * w.output * sizeof(float)) +
+               align256(uint64_t(narrow_counters(m, w)) * 4);
     const Handoff h = gemm_handoff(m, w);
     const uint32_t s = wide_splits(m, w);
     return afrag_bytes(w, m) + (h.x ? align256(handoff_bytes(h.x)) + align256(uint64_t(h.x) * 4) : 0) +
@@ -209,11 +233,10 @@ uint32_t gemm_launch_count(const DeviceWeights& w, uint64_t rows) {
     for (uint64_t r0 = 0; r0 < rows; r0 += pass) {
         const uint64_t m = rows - r0 < pass ? rows - r0 : pass;
         n += 2;
-        if (!gemm_wide(m, w) && narrow_splits(w) > 1) ++n;   // plane fold
+        n += pass_folds(m, w);
         if (gemm_wide(m, w)) {
             const WideSplit sp = wide_split(m, w);
             n += sp.full && sp.half;
-            if (wide_splits(m, w) > 1) ++n;   // plane fold
         }
     }
     return n;

@@ -24,6 +24,9 @@ WideSplit wide_split(uint64_t m, const DeviceWeights& w);
 bool gemm_wide(uint64_t m, const DeviceWeights& w);
 uint32_t wide_splits(uint64_t m, const DeviceWeights& w);
 uint32_t narrow_splits(const DeviceWeights& w);
+uint32_t narrow_rows(uint64_t m, const DeviceWeights& w);
+uint32_t narrow_counters(uint64_t m, const DeviceWeights& w);
+bool pass_folds(uint64_t m, const DeviceWeights& w);
 Handoff gemm_handoff(uint64_t m, const DeviceWeights& w);
 uint64_t handoff_bytes(uint32_t x);
 uint64_t pass_workspace(const DeviceWeights& w, uint64_t m);
