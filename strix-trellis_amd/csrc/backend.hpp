@@ -93,6 +93,10 @@ struct LinearCall {
     uint32_t handoff_poll_limit = 4096;
     // Single-launch GEMV: poll rounds of a finisher before it gives up.
     uint32_t gemv_poll_limit = GEMV_DEFAULT_POLL_LIMIT;
+    // Grouped GEMV of two groups: when set, hidden[r][n] = SwiGLU(y of group 0,
+    // y of group 1) follows the product (row stride in elements).
+    float* swiglu_hidden = nullptr;
+    uint64_t swiglu_row_stride = 0;
 };
 
 // Generic GEMV (rows 1..8): core kernel + finishing kernel, no counters.

@@ -2,6 +2,7 @@
 // workspace sizes are in policy.cpp); plus the finishing kernels and the
 // diagnostic stage kernels.
 #include "gemv_kernel.hpp"
+#include "moe.hpp"
 
 namespace stx {
 
@@ -176,10 +177,16 @@ hipError_t launch_gemv_grouped(const DeviceWeights& geometry, const GroupWeights
     GemvLaunch l = make_launch(geometry, table, groups, call, x_group_stride, y_group_stride,
                                static_cast<float*>(call.workspace), state, stream);
     hipError_t e = gemv_table[geometry.bits - 1](l);
-    if (e != hipSuccess || state || l.args.splits == 1) return e;
-    hipLaunchKernelGGL(gemv_finish_kernel, dim3(geometry.output / 128, 1, groups), dim3(GEMV_THREADS), 0,
-                       stream, l.args);
-    return hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (!state && l.args.splits > 1) {
+        hipLaunchKernelGGL(gemv_finish_kernel, dim3(geometry.output / 128, 1, groups), dim3(GEMV_THREADS), 0,
+                           stream, l.args);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    if (!call.swiglu_hidden) return hipSuccess;
+    if (groups != 2 || call.y_row_stride != geometry.output) return hipErrorInvalidValue;
+    return launch_swiglu_rows(call.y, call.y + y_group_stride, call.swiglu_hidden, call.swiglu_row_stride,
+                              uint32_t(call.rows), geometry.output, stream);
 }
 
 using GemvOwnerDispatch = hipError_t (*)(const GemvLaunch&);

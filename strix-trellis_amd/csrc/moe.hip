@@ -114,6 +114,21 @@ __global__ __launch_bounds__(256) void moe_swiglu_kernel(const float* g, const f
     if (i < n) h[i] = moe_swiglu(g[i], u[i]);
 }
 
+__global__ __launch_bounds__(256) void swiglu_rows_kernel(const float* g, const float* u, float* h, uint64_t h_stride,
+                                                          uint32_t width) {
+    const uint32_t n = blockIdx.x * 256 + threadIdx.x, r = blockIdx.y;
+    const uint64_t i = uint64_t(r) * width + n;
+    if (n < width) h[uint64_t(r) * h_stride + n] = moe_swiglu(g[i], u[i]);
+}
+
+hipError_t launch_swiglu_rows(const float* g, const float* u, float* h, uint64_t h_stride, uint32_t rows,
+                              uint32_t width, hipStream_t stream) {
+    if (!rows || !width) return hipSuccess;
+    hipLaunchKernelGGL(swiglu_rows_kernel, dim3((width + 255) / 256, rows), dim3(256), 0, stream, g, u, h, h_stride,
+                       width);
+    return hipGetLastError();
+}
+
 hipError_t launch_moe_swiglu(const float* g, const float* u, float* h, uint64_t n, hipStream_t stream) {
     if (!n) return hipSuccess;
     const uint64_t blocks = (n + 255) / 256;

@@ -95,5 +95,8 @@ uint64_t moe_gate_up_partial_floats(uint32_t routes, uint32_t I, uint32_t H);
 uint64_t moe_down_partial_floats(uint32_t routes, uint32_t I, uint32_t H);   // plain plans' planes
 // Diagnostic: h[i] = SwiGLU(g[i], u[i]) with the block's activation arithmetic.
 hipError_t launch_moe_swiglu(const float* g, const float* u, float* h, uint64_t n, hipStream_t stream);
+// The same over [rows][width] g and u (contiguous) into rows of stride h_stride.
+hipError_t launch_swiglu_rows(const float* g, const float* u, float* h, uint64_t h_stride, uint32_t rows,
+                              uint32_t width, hipStream_t stream);
 
 }  // namespace stx
