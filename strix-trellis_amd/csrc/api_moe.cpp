@@ -483,7 +483,9 @@ strix_status strix_tp_moe_plan_submit(strix_tp_moe_plan p) {
     const strix_status s = plan_ok(p);
     if (s != STRIX_SUCCESS) return s;
     hipError_t e = stx::launch_moe_gate_up(p->args, p->stream);
-    if (e == hipSuccess) e = stx::launch_moe_down(p->args, p->stream);
+    stx::MoeArgs down = p->args;
+    down.listed = 1;   // the gate/up launch of this submission resolves the groups
+    if (e == hipSuccess) e = stx::launch_moe_down(down, p->stream);
     return status_of(e);
 }
 

@@ -29,7 +29,8 @@ static bool moe_args_ok(const MoeArgs& a) {
 // its token is invalid, and the gate/up launch reads only valid tokens' routes.
 __global__ __launch_bounds__(GEMV_THREADS) void moe_input_kernel(const float* x, const uint32_t* ids,
                                                                  const MoeExpert* bank, uint32_t topk,
-                                                                 uint32_t bank_count, uint32_t x_stride, MoeArgs args) {
+                                                                 uint32_t bank_count, uint32_t x_stride, uint32_t routes,
+                                                                 MoeArgs args) {
     // Everything its first loads need is preloaded (scalar arguments).
     MoeArgs a = args;
     a.x = x;
@@ -40,6 +41,35 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_input_kernel(const float* x,
     a.x_stride = x_stride;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint32_t j = blockIdx.y, b = blockIdx.x * GEMV_WAVES + uint32_t(w);
+    if (j == routes) {
+        // One wave past the routes resolves them and writes the group list, one
+        // lane per route: a leading route writes its group's entry at its rank, slot
+        // 0 of an invalid token that token's NaN entry behind the groups, and the
+        // lanes of the ranks left over empty entries.
+        if (b != 0) return;
+        __shared__ uint32_t table[MOE_MAX_BANK];
+        const MoeLeaders l = moe_leaders(a, table);
+        const uint64_t bit = 1ull << lane, below = bit - 1;
+        uint64_t members = 0;
+        for (uint32_t t = 0; t < routes; ++t)
+            members |= uint64_t(__builtin_amdgcn_readlane(int(l.rt.id), int(t)) == int(l.rt.id)) << t;
+        members &= l.rt.valid;
+        const uint32_t groups = uint32_t(__builtin_popcountll(l.leaders));
+        const uint32_t used = groups + uint32_t(__builtin_popcountll(l.firsts));
+        auto* list = reinterpret_cast<MoeGroupEntry*>(reinterpret_cast<char*>(a.a_gu) + moe_group_list_offset(routes, a.I));
+        if (l.leaders & bit) {
+            const MoeExpert& ex = a.bank[l.rt.id];
+            list[__builtin_popcountll(l.leaders & below)] =
+                MoeGroupEntry{members, members & l.rt.nonzero, l.rt.id, uint32_t(lane), 1u, -1,
+                              {ex.gate.trellis, ex.up.trellis, ex.down.trellis}};
+        }
+        if (l.firsts & bit)
+            list[groups + uint32_t(__builtin_popcountll(l.firsts & below))] =
+                MoeGroupEntry{0, 0, 0, 0, 0u, int32_t(uint32_t(lane) / a.topk), {nullptr, nullptr, nullptr}};
+        if (uint32_t(lane) >= used && uint32_t(lane) < routes)
+            list[lane] = MoeGroupEntry{0, 0, 0, 0, 0u, -1, {nullptr, nullptr, nullptr}};
+        return;
+    }
     if (b >= a.I / 128) return;
     const float* xr = a.x + uint64_t(j / a.topk) * a.x_stride + 128 * b;
     const float x0 = ld_global(xr + lane), x1 = ld_global(xr + lane + 64);   // issued ahead of the id's round trip
@@ -62,9 +92,9 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_input_kernel(const float* x,
 hipError_t launch_moe_gate_up(const MoeArgs& a, hipStream_t stream) {
     if (!moe_args_ok(a) || !a.a_gu) return hipErrorInvalidValue;
     if (a.x_stride > 0xFFFFFFFFull) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(moe_input_kernel, dim3((a.I / 128 + GEMV_WAVES - 1) / GEMV_WAVES, a.rows * a.topk),
+    hipLaunchKernelGGL(moe_input_kernel, dim3((a.I / 128 + GEMV_WAVES - 1) / GEMV_WAVES, a.rows * a.topk + 1),
                        dim3(GEMV_THREADS), 0, stream, a.x, a.ids, a.bank, a.topk, a.bank_count,
-                       uint32_t(a.x_stride), a);
+                       uint32_t(a.x_stride), a.rows * a.topk, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return gate_up_table[a.gate_bits - 2](a, stream);
@@ -80,6 +110,7 @@ hipError_t launch_moe_down(const MoeArgs& a, hipStream_t stream) {
 hipError_t launch_moe_down_core(const MoeArgs& a, MoeDownMode mode, hipStream_t stream) {
     if (!moe_args_ok(a) || (mode != kMoeDownCore && mode != kMoeDownRouteCore)) return hipErrorInvalidValue;
     MoeArgs b = a;
+    b.listed = 0;
     b.down_mode = mode;
     return down_table[a.down_bits - 2](b, stream);
 }

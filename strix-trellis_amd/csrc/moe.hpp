@@ -12,9 +12,10 @@
 //
 // Both launches take the routes as device buffers [rows][k] of bank indices;
 // the plans built from host routes upload them once.  The union of experts is
-// resolved inside the kernels: the first valid occurrence of an expert in
-// row-major route order leads its group, every other occurrence's workgroups
-// exit, so each expert's weights are streamed once for all its tokens.
+// resolved on the device: the first valid occurrence of an expert in row-major
+// route order leads its group, so each expert's weights are streamed once for
+// all its tokens.  The gate/up's input launch lists the groups; a submission's
+// down reads that list, a down launch of its own resolves the routes itself.
 #pragma once
 #include "backend.hpp"
 
@@ -46,6 +47,17 @@ struct MoeArgs {
     uint32_t gate_bits, up_bits, down_bits;
     float alpha, beta;
     uint32_t down_mode;       // MoeDownMode of a down launch
+    uint32_t listed;          // down launch: the submission's gate/up has written the group list
+};
+
+// One workgroup rank's expert group, as moe_input_kernel resolves it for the
+// launches that follow in the submission (list of rows*k entries behind the
+// core inputs in a_gu): the fields of MoeGroup and the expert's weights.
+struct alignas(64) MoeGroupEntry {
+    uint64_t members, active;
+    uint32_t expert, route, leader;
+    int32_t nan_row;
+    const uint32_t* trellis[3];   // gate, up, down
 };
 
 // What a down launch does.  The staged modes write the per-split partial
@@ -83,8 +95,12 @@ uint64_t moe_counter_words(uint32_t rows, uint32_t routes, uint32_t I, uint32_t 
 // SwiGLU (a second launch that reads them).
 hipError_t launch_moe_gate_up(const MoeArgs& a, hipStream_t stream);
 hipError_t launch_moe_down(const MoeArgs& a, hipStream_t stream);
-// Bytes of a_gu for `routes` routes of input width I.
-constexpr uint64_t moe_core_input_bytes(uint32_t routes, uint32_t I) { return uint64_t(routes) * 2 * I * 2; }
+// Bytes of a_gu for `routes` routes of input width I: the core inputs, then the
+// group list.
+constexpr uint64_t moe_group_list_offset(uint32_t routes, uint32_t I) { return uint64_t(routes) * 2 * I * 2; }
+constexpr uint64_t moe_core_input_bytes(uint32_t routes, uint32_t I) {
+    return moe_group_list_offset(routes, I) + uint64_t(routes) * sizeof(MoeGroupEntry);
+}
 // Staged down: the core alone in `mode` (kMoeDownCore or kMoeDownRouteCore),
 // and the finish alone, which folds the planes p_d as they are in memory
 // (ascending split from +0, output stage, ordered score-weighted slot sum,

@@ -5,13 +5,15 @@
 // the matrix-core dot, LDS wave fold, coherent partial planes, last-arrival
 // finish) with routed rows instead of a fixed row range:
 //
-//   gate/up : grid (H/128, s_gu, rows*k), 256 threads.  Workgroup (c, s, r)
+//   gate/up : grid (H/128, 2 s_gu, rows*k), 256 threads.  Workgroup (c, 2s + p, r)
 //             takes the r-th expert group (its leader is the first valid
-//             occurrence of the expert in route order).  It gathers the group's
-//             non-zero-score token rows of X, streams gate AND up tiles of
-//             column group c over input split s and writes both partial
-//             planes; the last split to arrive folds them, applies both output
-//             stages and SwiGLU and writes hidden[r, slot, 128c .. 128c+127].
+//             occurrence of the expert in route order), as the input launch
+//             ahead has listed it.  It pulls the group's non-zero-score rows
+//             of core inputs, streams the tiles of projection p (0 gate, 1 up)
+//             of column group c over input split s and writes its partial
+//             plane; the last of the 2 s_gu to arrive folds both projections,
+//             applies both output stages and SwiGLU and writes hidden[r, slot,
+//             128c .. 128c+127].
 //   down    : grid (I/128, s_d, rows*k).  The group leader streams the down
 //             tiles once for all its rows (input = hidden of each row) and
 //             writes one plane per row; every workgroup of a group then
@@ -135,43 +137,51 @@ __device__ __forceinline__ void moe_keep_routes(const MoeRoutes& rt, uint32_t* w
 // first and spread evenly over the CUs, instead of sitting wherever their
 // routes happen to lead.  Ranks past the groups take the
 // invalid tokens in order (there are at least as many: an invalid token's k
-// routes lead nothing).  One lane per route, in one wave (moe_group_shared).
+// routes lead nothing).  One lane per route, in one wave.
 //
 // A route leads its group when no lower valid route selects the same expert.
 // The leaders come from a table of each expert's first valid route (an LDS
 // minimum over the valid lanes), so the resolution costs the same for every
 // rank; the r-th leader in route order is the r-th set bit of their ballot.
 // `table` is MOE_MAX_BANK words of LDS that nothing else uses meanwhile.
-__device__ __forceinline__ MoeGroup moe_resolve(const MoeArgs& a, uint32_t rank, uint32_t* table,
-                                                uint32_t* keep = nullptr) {
+struct MoeLeaders {
+    MoeRoutes rt;
+    uint64_t leaders, firsts;   // leading routes; slot 0 of each invalid token
+};
+__device__ __forceinline__ MoeLeaders moe_leaders(const MoeArgs& a, uint32_t* table) {
     const int lane = threadIdx.x & 63;
     const uint32_t k = a.topk, n = a.rows * k;
     const bool live = uint32_t(lane) < n;
     const uint32_t slot = uint32_t(lane) % k;
     const MoeRoutes rt = moe_routes(a);
-    if (keep) moe_keep_routes(rt, keep);
-    const uint32_t id = rt.id;
     const bool tv = (rt.valid >> lane) & 1;   // valid implies id < bank_count <= MOE_MAX_BANK
     for (uint32_t i = uint32_t(lane); i < a.bank_count; i += 64) table[i] = ~0u;
     __builtin_amdgcn_wave_barrier();   // lanes exchange through the table: keep the three steps in order
-    if (tv) __hip_atomic_fetch_min(table + id, uint32_t(lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (tv) __hip_atomic_fetch_min(table + rt.id, uint32_t(lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     __builtin_amdgcn_wave_barrier();
-    const bool leads = tv && __hip_atomic_load(table + id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) ==
+    const bool leads = tv && __hip_atomic_load(table + rt.id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) ==
                                  uint32_t(lane);
-    const uint64_t leaders = __ballot(leads);
-    const uint32_t groups = uint32_t(__builtin_popcountll(leaders));
+    return {rt, __ballot(leads), __ballot(live && slot == 0 && !tv)};
+}
+__device__ __forceinline__ MoeGroup moe_rank_group(const MoeLeaders& l, uint32_t k, uint32_t rank) {
+    const uint32_t groups = uint32_t(__builtin_popcountll(l.leaders));
     if (rank < groups) {
-        const uint32_t lead = moe_nth_route(leaders, int(rank));
-        const uint32_t e = uint32_t(__builtin_amdgcn_readlane(int(id), int(lead)));
-        const uint64_t members = __ballot(id == e) & rt.valid;
-        return {members, members & rt.nonzero, e, lead, true, -1};
+        const uint32_t lead = moe_nth_route(l.leaders, int(rank));
+        const uint32_t e = uint32_t(__builtin_amdgcn_readlane(int(l.rt.id), int(lead)));
+        const uint64_t members = __ballot(l.rt.id == e) & l.rt.valid;
+        return {members, members & l.rt.nonzero, e, lead, true, -1};
     }
     // Invalid tokens: slot 0 of each row whose routes are not valid.
-    const uint64_t firsts = __ballot(live && slot == 0 && !tv);
     int nan_row = -1;
-    if (rank - groups < uint32_t(__builtin_popcountll(firsts)))
-        nan_row = int(moe_nth_route(firsts, int(rank - groups)) / k);
+    if (rank - groups < uint32_t(__builtin_popcountll(l.firsts)))
+        nan_row = int(moe_nth_route(l.firsts, int(rank - groups)) / k);
     return {0, 0, 0, 0, false, nan_row};
+}
+__device__ __forceinline__ MoeGroup moe_resolve(const MoeArgs& a, uint32_t rank, uint32_t* table,
+                                                uint32_t* keep = nullptr) {
+    const MoeLeaders l = moe_leaders(a, table);
+    if (keep) moe_keep_routes(l.rt, keep);
+    return moe_rank_group(l, a.topk, rank);
 }
 
 // Route-alone resolution (the reference-core down): workgroup rank j takes
@@ -230,6 +240,25 @@ __device__ __forceinline__ MoeGroup moe_group_shared(const MoeArgs& a, uint32_t 
     const MoeGroup g = {uint64_t(v[0]) | (uint64_t(v[1]) << 32), uint64_t(v[2]) | (uint64_t(v[3]) << 32), v[4], v[5],
                         v[6] != 0, int(v[7])};
     return moe_uniform(g);
+}
+
+// The group list entry of this rank, read with scalar loads (the list is
+// written by an earlier launch, and nothing of this launch changes it).  Without
+// the list every workgroup resolved the routes itself: the ids' round trip, an
+// LDS table and a few hundred issue slots, a barrier, then the bank entry's.
+__device__ __forceinline__ MoeGroupEntry moe_listed(const void* list, uint32_t rank) {
+    typedef const __attribute__((address_space(4))) uint64_t* scalar_ptr;
+    const scalar_ptr q = scalar_ptr(reinterpret_cast<uintptr_t>(list) + uint64_t(rank) * sizeof(MoeGroupEntry));
+    const uint64_t v[7] = {q[0], q[1], q[2], q[3], q[4], q[5], q[6]};
+    MoeGroupEntry e;
+    e.members = v[0];
+    e.active = v[1];
+    e.expert = uint32_t(v[2]);
+    e.route = uint32_t(v[2] >> 32);
+    e.leader = uint32_t(v[3]);
+    e.nan_row = int32_t(v[3] >> 32);
+    for (int i = 0; i < 3; ++i) e.trellis[i] = reinterpret_cast<const uint32_t*>(uintptr_t(v[4 + i]));
+    return e;
 }
 
 // Fold `splits` planes of two sets p and q (stride between splits `step`
@@ -291,8 +320,8 @@ constexpr int MOE_RING_GU = 3;
 constexpr int MOE_RING_D = 4;
 // LDS: the FP16 activations live until the main loop ends, the wave partials
 // only after it, so both share one buffer.
-constexpr int MOE_GU_ACT_BYTES = 2 * MOE_MAX_RT * MOE_GU_MAX_BPS * 16 * 2;
-constexpr int MOE_GU_RED_BYTES = GEMV_WAVES * 2 * MOE_MAX_RT * 128 * 4;
+constexpr int MOE_GU_ACT_BYTES = MOE_MAX_RT * MOE_GU_MAX_BPS * 16 * 2;
+constexpr int MOE_GU_RED_BYTES = GEMV_WAVES * MOE_MAX_RT * 128 * 4;
 constexpr int MOE_D_ACT_BYTES = MOE_MAX_RT * MOE_D_MAX_BPS * 16 * 2;
 constexpr int MOE_D_RED_BYTES = GEMV_WAVES * MOE_MAX_RT * 128 * 4;
 static_assert(MOE_GU_ACT_BYTES >= int(MOE_MAX_BANK * 4) && MOE_D_ACT_BYTES >= int(MOE_MAX_BANK * 4),
@@ -331,92 +360,96 @@ __device__ __forceinline__ void moe_input_stage(int w, int units, const InputLoa
 }
 
 // ---------------------------------------------------------------------------
-// Gate/up core of one workgroup: NP = 2 projections sharing the routed rows.
+// Gate/up core of one workgroup: projection p (0 gate, 1 up) of one column
+// group and input split.  Bound by the decode's VALU on the CU with the most
+// workgroups: with both projections in one workgroup, one token's six experts of
+// 5120 <-> 1152 gave 270 workgroups for 256 CUs, and 14 CUs took twice the time
+// of the rest.  One projection each halves the unit (same chains, same bits).
+// With the group list (below) the block took, us of 1 / 8 tokens: 5120 <-> 1152
+// top-6 42.3 / 105.6 -> 35.7 / 97.7, 4096 <-> 1536 top-8 46.0 / 124.5 -> 40.4 / 121.5
+// (without the list 36.7 / 100.1 and 40.7 / 122.5).
 // ---------------------------------------------------------------------------
-template <int KG, int KU, int RT>
-__device__ __forceinline__ void moe_gate_up_core(const MoeArgs& a, const MoeExpert& ex, uint32_t c, uint32_t split,
-                                                 uint64_t active, int nrows, _Float16* act, float* red) {
+template <int K, int RT>
+__device__ __forceinline__ void moe_gate_up_core(const MoeArgs& a, const char* trellis, uint32_t p, uint32_t c,
+                                                 uint32_t split, uint64_t active, int nrows, _Float16* act,
+                                                 float* red) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int jt = lane >> 3, g = lane & 7;
     const uint32_t bps = a.bps_gu, a0 = split * bps;
     const uint32_t act_row = bps * 16;
-    constexpr uint32_t tg = 32u * KG, tu = 32u * KU;
-    const uint32_t rbg = (a.H >> 4) * tg, rbu = (a.H >> 4) * tu;
-    const auto rg = make_rsrc(moe_first_ptr(ex.gate.trellis) + uint64_t(a0) * rbg, bps * rbg);
-    const auto ru = make_rsrc(moe_first_ptr(ex.up.trellis) + uint64_t(a0) * rbu, bps * rbu);
-    const uint32_t og = (8u * c + jt) * tg + g * 4u * KG, ou = (8u * c + jt) * tu + g * 4u * KU;
+    constexpr uint32_t tb = 32u * K;
+    const uint32_t rb = (a.H >> 4) * tb;
+    const auto rs = make_rsrc(trellis + uint64_t(a0) * rb, bps * rb);
+    const uint32_t lo = (8u * c + jt) * tb + g * 4u * K;
     const int nb = int(bps) / GEMV_WAVES;
     constexpr uint32_t kOut = 0x80000000u;
-    auto offg = [&](int t) -> uint32_t { return t < nb ? (w + GEMV_WAVES * t) * rbg + og : kOut; };
-    auto offu = [&](int t) -> uint32_t { return t < nb ? (w + GEMV_WAVES * t) * rbu + ou : kOut; };
+    auto off = [&](int t) -> uint32_t { return t < nb ? (w + GEMV_WAVES * t) * rb + lo : kOut; };
 
     // Core inputs of the split's channels, computed once per route by
     // moe_input_kernel (every column group of an expert used to recompute
-    // them): one 256-byte unit per (projection, row, 128-block), 4 bytes per
-    // lane, straight into LDS by DMA, no registers in flight.  Issued before
-    // the weight prefetch: vector loads complete in issue order, so loads
-    // issued after the chunks would wait for the chunks' HBM round trip.
-    // Wave w takes 128-blocks w, w + 4, ... of every row and projection
-    // (scalar loops, no divisions).
+    // them): one 256-byte unit per (row, 128-block), 4 bytes per lane, straight
+    // into LDS by DMA, no registers in flight.  Issued before the weight
+    // prefetch: vector loads complete in issue order, so loads issued after the
+    // chunks would wait for the chunks' HBM round trip.  Wave w takes 128-blocks
+    // w, w + 4, ... of every row (scalar loops, no divisions).
     const int hblocks = int(bps) / 8;
-    const auto ars = make_rsrc(a.a_gu, uint32_t(moe_core_input_bytes(a.rows * a.topk, a.I)));
+    const auto ars = make_rsrc(a.a_gu, uint32_t(moe_group_list_offset(a.rows * a.topk, a.I)));
     uint64_t left = active;
     for (int i = 0; i < nrows; ++i) {   // wave-uniform
         const uint32_t j = uint32_t(__builtin_ctzll(left));
         left &= left - 1;
-        for (int p = 0; p < 2; ++p)
-            for (int hb = w; hb < hblocks; hb += GEMV_WAVES) {
-                const uint32_t src = ((j * 2 + uint32_t(p)) * a.I + a0 * 16 + uint32_t(hb) * 128) * 2;
-                _Float16* dst = act + (p * MOE_MAX_RT + i) * act_row + hb * 128;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (__attribute__((address_space(3))) void*)dst, 4,
-                                                         uint32_t(lane) * 4u, src, 0, 0);
-            }
+        for (int hb = w; hb < hblocks; hb += GEMV_WAVES) {
+            const uint32_t src = ((j * 2 + p) * a.I + a0 * 16 + uint32_t(hb) * 128) * 2;
+            _Float16* dst = act + i * act_row + hb * 128;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (__attribute__((address_space(3))) void*)dst, 4,
+                                                     uint32_t(lane) * 4u, src, 0, 0);
+        }
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    Chunk<KG> cg[MOE_RING_GU];
-    Chunk<KU> cu[MOE_RING_GU];
+    Chunk<K> ring[MOE_RING_GU];
 #pragma unroll
-    for (int u = 0; u < MOE_RING_GU; ++u) {
-        load_chunk(cg[u], rg, offg(u));
-        load_chunk(cu[u], ru, offu(u));
-    }
+    for (int u = 0; u < MOE_RING_GU; ++u) load_chunk(ring[u], rs, off(u));
     __builtin_amdgcn_sched_barrier(0);
-    // The compiler does not see the DMAs' LDS side: wait for them by count
-    // (the 2 x MOE_RING_GU chunk loads, one instruction each at K <= 3, were
-    // issued after them), then the barrier makes every wave's units visible.
-    static_assert(KG <= 3 && KU <= 3, "one load instruction per chunk");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * MOE_RING_GU) : "memory");
+    // The compiler does not see the DMAs' LDS side: wait for them by count (the
+    // MOE_RING_GU chunk loads, one instruction each at K <= 3, were issued after
+    // them), then the barrier makes every wave's units visible.
+    static_assert(K <= 3, "one load instruction per chunk");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MOE_RING_GU) : "memory");
     // Rows past nrows stay unused: rows nrows..RT-1 hold stale LDS, their
     // columns of the products are independent of the others, and the fold
     // below reads only rows < nrows.
     __syncthreads();
 
-    MfmaAcc<RT> accg, accu;
-    mfma_acc_zero(accg);
-    mfma_acc_zero(accu);
+    MfmaAcc<RT> acc;
+    mfma_acc_zero(acc);
     const bool first = g == 0;
     for (int t = 0; t < nb; t += MOE_RING_GU) {
 #pragma unroll
         for (int u = 0; u < MOE_RING_GU; ++u) {
             if (t + u < nb) {
-                const int blk = w + GEMV_WAVES * (t + u);
                 half2_t wq[4][4];
-                link_chunk(cg[u], first);
-                decode_chunk<KG, CB_MUL1>(cg[u], wq);
-                mfma_dot_block<RT>(wq, act + blk * 16, act_row, accg);
-                link_chunk(cu[u], first);
-                decode_chunk<KU, CB_MUL1>(cu[u], wq);
-                mfma_dot_block<RT>(wq, act + MOE_MAX_RT * act_row + blk * 16, act_row, accu);
+                link_chunk(ring[u], first);
+                decode_chunk<K, CB_MUL1>(ring[u], wq);
+                mfma_dot_block<RT>(wq, act + (w + GEMV_WAVES * (t + u)) * 16, act_row, acc);
             }
-            load_chunk(cg[u], rg, offg(t + u + MOE_RING_GU));
-            load_chunk(cu[u], ru, offu(t + u + MOE_RING_GU));
+            load_chunk(ring[u], rs, off(t + u + MOE_RING_GU));
         }
     }
     __syncthreads();   // every wave is done with act before red overwrites it
-    mfma_partials<RT>(accg, red + (w * 2 + 0) * MOE_MAX_RT * 128);
-    mfma_partials<RT>(accu, red + (w * 2 + 1) * MOE_MAX_RT * 128);
+    mfma_partials<RT>(acc, red + w * MOE_MAX_RT * 128);
     __syncthreads();
+}
+
+// The row template of the group's routes.
+template <int K>
+__device__ __forceinline__ void moe_gate_up_rows(const MoeArgs& a, const char* trellis, uint32_t p, uint32_t c,
+                                                 uint32_t split, uint64_t active, int nrows, _Float16* act,
+                                                 float* red) {
+    if (nrows <= 1) moe_gate_up_core<K, 1>(a, trellis, p, c, split, active, nrows, act, red);
+    else if (nrows <= 2) moe_gate_up_core<K, 2>(a, trellis, p, c, split, active, nrows, act, red);
+    else if (nrows <= 4) moe_gate_up_core<K, 4>(a, trellis, p, c, split, active, nrows, act, red);
+    else moe_gate_up_core<K, 8>(a, trellis, p, c, split, active, nrows, act, red);
 }
 
 // Waves per SIMD the MoE kernels ask the register allocator for: five
@@ -424,46 +457,40 @@ __device__ __forceinline__ void moe_gate_up_core(const MoeArgs& a, const MoeExpe
 // projection would spill at five).
 constexpr int moe_waves_per_eu(int bits_sum, int projections) { return bits_sum <= 2 * projections ? 5 : 4; }
 
-// LDS is the one activation / partial buffer and nothing else (32 KiB at the
-// largest split), so that five workgroups fit a CU.
+// LDS is the one activation / partial buffer (16 KiB at the largest split).
 template <int KG, int KU>
-__global__ __launch_bounds__(GEMV_THREADS) __attribute__((amdgpu_waves_per_eu(moe_waves_per_eu(KG + KU, 2))))
-void moe_gate_up_kernel(const uint32_t* ids, const float* scores, const MoeExpert* bank, uint32_t rows_topk,
-                        uint32_t bank_count, MoeArgs args) {
-    // The route resolution's inputs and the bank come as scalar arguments, so
-    // the dispatcher preloads them into SGPRs and the first loads (the routes)
-    // wait for no argument load (the rest of MoeArgs is needed after them).
+__global__ __launch_bounds__(GEMV_THREADS) __attribute__((amdgpu_waves_per_eu(moe_waves_per_eu(KG > KU ? KG : KU, 1))))
+void moe_gate_up_kernel(const MoeGroupEntry* list, const MoeExpert* bank, MoeArgs args) {
+    // The group list comes as a scalar argument, so the dispatcher preloads it
+    // and the first load (the rank's entry) waits for no argument load.
     MoeArgs a = args;
-    a.ids = ids;
-    a.scores = scores;
     a.bank = bank;
-    a.rows = rows_topk & 0xFFFFu;
-    a.topk = rows_topk >> 16;
-    a.bank_count = bank_count;
     __shared__ __align__(16) unsigned char lds[moe_max(MOE_GU_ACT_BYTES, MOE_GU_RED_BYTES)];
     _Float16* act = reinterpret_cast<_Float16*>(lds);
     float* red = reinterpret_cast<float*>(lds);
-    __shared__ uint32_t group_slot[8];
-    const uint32_t c = blockIdx.x, split = blockIdx.y;
+    const uint32_t c = blockIdx.x, split = blockIdx.y >> 1, p = blockIdx.y & 1;
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const MoeGroup grp = moe_group_shared(a, blockIdx.z, group_slot, reinterpret_cast<uint32_t*>(lds));
+    const MoeGroupEntry grp = moe_listed(list, blockIdx.z);
     if (!grp.leader || !grp.active) return;
     const uint32_t route = grp.route;
     const uint64_t active = grp.active;
     const int nrows = __builtin_popcountll(active);
     const MoeExpert& ex = a.bank[grp.expert];
-    if (nrows <= 1) moe_gate_up_core<KG, KU, 1>(a, ex, c, split, active, nrows, act, red);
-    else if (nrows <= 2) moe_gate_up_core<KG, KU, 2>(a, ex, c, split, active, nrows, act, red);
-    else if (nrows <= 4) moe_gate_up_core<KG, KU, 4>(a, ex, c, split, active, nrows, act, red);
-    else moe_gate_up_core<KG, KU, 8>(a, ex, c, split, active, nrows, act, red);
+    const char* trellis = reinterpret_cast<const char*>(p ? grp.trellis[1] : grp.trellis[0]);
+    if constexpr (KG == KU) {
+        moe_gate_up_rows<KG>(a, trellis, p, c, split, active, nrows, act, red);
+    } else {
+        if (p) moe_gate_up_rows<KU>(a, trellis, p, c, split, active, nrows, act, red);
+        else moe_gate_up_rows<KG>(a, trellis, p, c, split, active, nrows, act, red);
+    }
 
     // Wave fold in wave order -> planes [route][split][proj][H].
     const uint32_t S = a.s_gu, H = a.H;
-    for (int idx = tid; idx < 2 * nrows * 128; idx += GEMV_THREADS) {
-        const int n = idx & 127, pr = idx >> 7, p = pr & 1, i = pr >> 1;
-        float v = red[((0 * 2 + p) * MOE_MAX_RT + i) * 128 + n];
+    for (int idx = tid; idx < nrows * 128; idx += GEMV_THREADS) {
+        const int n = idx & 127, i = idx >> 7;
+        float v = red[i * 128 + n];
 #pragma unroll
-        for (int ww = 1; ww < GEMV_WAVES; ++ww) v = v + red[((ww * 2 + p) * MOE_MAX_RT + i) * 128 + n];
+        for (int ww = 1; ww < GEMV_WAVES; ++ww) v = v + red[(ww * MOE_MAX_RT + i) * 128 + n];
         const uint32_t j = moe_nth_route(active, i);
         store_coherent(a.p_gu + ((uint64_t(j) * S + split) * 2 + p) * H + 128 * c + n, v);
     }
@@ -471,7 +498,7 @@ void moe_gate_up_kernel(const uint32_t* ids, const float* scores, const MoeExper
     // The partials in LDS are consumed: word 0 carries the arrival result.
     uint32_t* counter = a.c_gu + uint64_t(route) * (H >> 7) + c;
     int* last = reinterpret_cast<int*>(lds);
-    if (tid == 0) *last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
+    if (tid == 0) *last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * S - 1;
     __syncthreads();
     if (!*last) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -508,8 +535,8 @@ void moe_gate_up_kernel(const uint32_t* ids, const float* scores, const MoeExper
 // Down core of one workgroup (one projection, rows = the group's active routes).
 // ---------------------------------------------------------------------------
 template <int K, int RT>
-__device__ __forceinline__ void moe_down_core(const MoeArgs& a, const MoeExpert& ex, uint32_t c, uint32_t split,
-                                              uint64_t active, int nrows, _Float16* act, float* red) {
+__device__ __forceinline__ void moe_down_core(const MoeArgs& a, const MoeExpert& ex, const char* trellis, uint32_t c,
+                                              uint32_t split, uint64_t active, int nrows, _Float16* act, float* red) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int jt = lane >> 3, g = lane & 7;
     // Blocks [a0, a0 + bps) of the input, inside 128-channel groups
@@ -520,7 +547,7 @@ __device__ __forceinline__ void moe_down_core(const MoeArgs& a, const MoeExpert&
     const uint32_t act_row = uint32_t(hblocks) * 128;
     constexpr uint32_t tb = 32u * K;
     const uint32_t rb = (a.I >> 4) * tb;
-    const auto rs = make_rsrc(moe_first_ptr(ex.down.trellis) + uint64_t(a0) * rb, bps * rb);
+    const auto rs = make_rsrc(trellis + uint64_t(a0) * rb, bps * rb);
     const uint32_t lo = (8u * c + jt) * tb + g * 4u * K;
     const int nb = (int(bps) - w + GEMV_WAVES - 1) / GEMV_WAVES;   // blocks w, w + 4, ... of the split
     constexpr uint32_t kOut = 0x80000000u;
@@ -649,7 +676,7 @@ __device__ __forceinline__ void moe_finish_token(const MoeArgs& a, uint32_t r, u
 template <int K>
 __global__ __launch_bounds__(GEMV_THREADS) __attribute__((amdgpu_waves_per_eu(moe_waves_per_eu(K, 1))))
 void moe_down_kernel(const uint32_t* ids, const float* scores, const MoeExpert* bank, uint32_t rows_topk,
-                     uint32_t bank_count, MoeArgs args) {
+                     uint32_t bank_count, const MoeGroupEntry* list, MoeArgs args) {
     // Preloaded resolution inputs, as in the gate/up kernel.
     MoeArgs a = args;
     a.ids = ids;
@@ -668,8 +695,25 @@ void moe_down_kernel(const uint32_t* ids, const float* scores, const MoeExpert* 
     __shared__ uint32_t group_slot[8];
     const bool staged = a.down_mode != kMoeDownFused;   // a kernel argument: uniform
     __shared__ uint32_t route_words[2 * MOE_MAX_ROUTES];
-    const MoeGroup grp = moe_group_shared(a, blockIdx.z, group_slot, reinterpret_cast<uint32_t*>(lds),
-                                          a.down_mode == kMoeDownRouteCore, route_words);
+    // Inside a submission (`list`) the rank's group comes from the gate/up's
+    // list; a down launch of its own resolves the routes as they are now.
+    MoeGroup grp;
+    const char* trellis = nullptr;
+    uint32_t id_l = 0, score_l = 0;
+    if (list) {
+        const MoeGroupEntry e = moe_listed(list, blockIdx.z);
+        grp = {e.members, e.active, e.expert, e.route, e.leader != 0, e.nan_row};
+        trellis = reinterpret_cast<const char*>(e.trellis[2]);
+        // The routes for a later token finish, in flight until the loop ends.
+        if (w == 0) {
+            const bool live = uint32_t(lane) < a.rows * k;
+            id_l = ld_global(a.ids + (live ? lane : 0));
+            score_l = __builtin_bit_cast(uint32_t, ld_global(a.scores + (live ? lane : 0)));
+        }
+    } else {
+        grp = moe_group_shared(a, blockIdx.z, group_slot, reinterpret_cast<uint32_t*>(lds),
+                               a.down_mode == kMoeDownRouteCore, route_words);
+    }
     if (!grp.leader) {
         // One workgroup per (invalid token, column group) writes its NaN row block.
         if (!staged && grp.nan_row >= 0 && split == 0 && tid < 128)
@@ -679,11 +723,12 @@ void moe_down_kernel(const uint32_t* ids, const float* scores, const MoeExpert* 
     const uint64_t active = grp.active, members = grp.members;
     const int nrows = __builtin_popcountll(active);
     const MoeExpert& ex = a.bank[grp.expert];
+    if (!list) trellis = moe_first_ptr(ex.down.trellis);
     if (nrows) {
-        if (nrows <= 1) moe_down_core<K, 1>(a, ex, c, split, active, nrows, act, red);
-        else if (nrows <= 2) moe_down_core<K, 2>(a, ex, c, split, active, nrows, act, red);
-        else if (nrows <= 4) moe_down_core<K, 4>(a, ex, c, split, active, nrows, act, red);
-        else moe_down_core<K, 8>(a, ex, c, split, active, nrows, act, red);
+        if (nrows <= 1) moe_down_core<K, 1>(a, ex, trellis, c, split, active, nrows, act, red);
+        else if (nrows <= 2) moe_down_core<K, 2>(a, ex, trellis, c, split, active, nrows, act, red);
+        else if (nrows <= 4) moe_down_core<K, 4>(a, ex, trellis, c, split, active, nrows, act, red);
+        else moe_down_core<K, 8>(a, ex, trellis, c, split, active, nrows, act, red);
         for (int idx = tid; idx < nrows * 128; idx += GEMV_THREADS) {
             const int n = idx & 127, i = idx >> 7;
             float v = red[(0 * MOE_MAX_RT + i) * 128 + n];
@@ -694,6 +739,10 @@ void moe_down_kernel(const uint32_t* ids, const float* scores, const MoeExpert* 
         }
     }
     if (staged) return;   // the planes are the staged core's result
+    if (list && w == 0) {
+        route_words[lane] = id_l;
+        route_words[MOE_MAX_ROUTES + lane] = score_l;
+    }
     moe_release();
     // One arrival per member route (one route per token), lanes in parallel.
     const uint32_t expected = k * S;
@@ -730,22 +779,26 @@ void moe_down_kernel(const uint32_t* ids, const float* scores, const MoeExpert* 
 #define STX_INSTANTIATE_MOE(KG)                                                                                   \
     template <>                                                                                                   \
     hipError_t moe_gate_up_dispatch<KG>(const MoeArgs& a, hipStream_t s) {                                        \
-        const dim3 grid(a.H / 128, a.s_gu, a.rows * a.topk);                                                      \
-        const uint32_t rk = a.rows | (a.topk << 16);                                                              \
+        const dim3 grid(a.H / 128, 2 * a.s_gu, a.rows * a.topk);                                                  \
+        const MoeGroupEntry* list = moe_group_list(a);                                                            \
         if (a.up_bits == 2)                                                                                       \
-            hipLaunchKernelGGL((moe_gate_up_kernel<KG, 2>), grid, dim3(GEMV_THREADS), 0, s, a.ids, a.scores,       \
-                               a.bank, rk, a.bank_count, a);                                                      \
+            hipLaunchKernelGGL((moe_gate_up_kernel<KG, 2>), grid, dim3(GEMV_THREADS), 0, s, list, a.bank, a);      \
         else                                                                                                      \
-            hipLaunchKernelGGL((moe_gate_up_kernel<KG, 3>), grid, dim3(GEMV_THREADS), 0, s, a.ids, a.scores,       \
-                               a.bank, rk, a.bank_count, a);                                                      \
+            hipLaunchKernelGGL((moe_gate_up_kernel<KG, 3>), grid, dim3(GEMV_THREADS), 0, s, list, a.bank, a);      \
         return hipGetLastError();                                                                                 \
     }                                                                                                             \
     template <>                                                                                                   \
     hipError_t moe_down_dispatch<KG>(const MoeArgs& a, hipStream_t s) {                                           \
         hipLaunchKernelGGL(moe_down_kernel<KG>, dim3(a.I / 128, a.s_d, a.rows * a.topk), dim3(GEMV_THREADS), 0, s, \
-                           a.ids, a.scores, a.bank, a.rows | (a.topk << 16), a.bank_count, a);                    \
+                           a.ids, a.scores, a.bank, a.rows | (a.topk << 16), a.bank_count,                        \
+                           a.listed ? moe_group_list(a) : nullptr, a);                                            \
         return hipGetLastError();                                                                                 \
     }
+
+inline const MoeGroupEntry* moe_group_list(const MoeArgs& a) {
+    return reinterpret_cast<const MoeGroupEntry*>(reinterpret_cast<const char*>(a.a_gu) +
+                                                  moe_group_list_offset(a.rows * a.topk, a.I));
+}
 
 template <int KG>
 hipError_t moe_gate_up_dispatch(const MoeArgs& a, hipStream_t s);
