@@ -30,9 +30,9 @@
 // Measured against 128 x 128 and 256 x 128 tiles of the same order (64 KiB of
 // LDS, two waves along each dimension; 320 workgroups on 5120^2 that multiplied
 // 128 rows whatever M was), calls, same bits: 5120^2 K5 M = 16 / 24 / 64 / 128 /
-// 200 24.5 / 24.6 / 27.6 / 30.9 / 40.7 -> 14.2 / 16.6 / 21.6 / 25.6 / 32.8 us, 4096
-// -> 12288 K6 29.1 / 29.4 / 32.0 / 35.7 / 49.7 -> 17.9 / 20.7 / 24.4 / 31.9 / 43.5 us,
-// 1152 -> 5120 K4 M = 16 / 128 25.0 / 30.3 -> 11.8 / 16.4 us; 5120 -> 1152 K4 M =
+// 200 24.5 / 24.6 / 27.6 / 30.9 / 40.7 -> 14.4 / 16.7 / 21.3 / 24.5 / 29.2 us, 4096
+// -> 12288 K6 29.1 / 29.4 / 32.0 / 35.7 / 49.7 -> 17.8 / 19.7 / 23.5 / 30.2 / 40.8 us,
+// 1152 -> 5120 K4 M = 16 / 128 25.0 / 30.3 -> 11.9 / 16.7 us; 5120 -> 1152 K4 M =
 // 512 / 4096 31.5 / 143.9 -> 27.0 / 127.9 us.
 //
 // MFMA 16x16x32 f16 operand layout (lane l, e = 0..7 / 0..3):
@@ -89,7 +89,8 @@ __host__ __device__ __forceinline__ uint64_t afrag_offset(uint32_t rb, uint32_t 
 constexpr int NARROW_BSTAGE_BYTES = 4 * 4 * 64 * 16;   // 4 tiles x 4 K32 steps x 64 lanes x 16 B
 
 template <int K, int CB, int TM, bool FOLD>
-__global__ __launch_bounds__(256) void gemm_narrow_kernel(const uint32_t* trellis, const _Float16* afrag, uint32_t input,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TM >= 8 ? 3 : 4)))
+void gemm_narrow_kernel(const uint32_t* trellis, const _Float16* afrag, uint32_t input,
                                                          uint32_t output, uint32_t splits, uint32_t rows,
                                                          GemmArgs args) {
     // What the first loads need comes as scalar arguments, preloaded into SGPRs.
@@ -103,7 +104,10 @@ __global__ __launch_bounds__(256) void gemm_narrow_kernel(const uint32_t* trelli
     a.afrag_bytes = uint64_t((rows + 15) / 16 * 16) * input * 2;
     constexpr int WM = TM >= 8 ? 4 : TM >= 2 ? 2 : 1, WN = 4 / WM;   // waves along M and N
     constexpr int RT = TM / WM, CT = 4 / WN;              // row and column tiles per wave
-    constexpr int D = 3;                                  // chunk ring: stages in flight
+    constexpr int D = RT >= 4 ? 2 : 3;                    // chunk ring: stages in flight
+    // A ring: K32 steps in flight.  Four (a whole stage) up to two row tiles per
+    // wave; with four, two, which leaves registers for three workgroups per CU.
+    constexpr int AD = RT >= 4 ? 2 : 4;
     __shared__ __align__(16) unsigned char smem[2 * NARROW_BSTAGE_BYTES];
     const int c = blockIdx.x, mb = blockIdx.y, split = blockIdx.z;
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -140,16 +144,28 @@ __global__ __launch_bounds__(256) void gemm_narrow_kernel(const uint32_t* trelli
         frag(std::integral_constant<int, 6>{}, 24);   // rows 8-15
     };
 
-    // A fragments of the wave's row tiles: slot k32 holds K32 step k32 of the
-    // current stage and is refilled with that step of the next stage once
-    // consumed.  Row tiles past the padded rows read out of range (zeros).
+    // A fragments of the wave's row tiles: slot t % AD holds K32 step t and is
+    // refilled with step t + AD once consumed.  Row tiles past the padded rows
+    // read out of range (zeros).
     const uint32_t rb0 = uint32_t(mb) * TM + uint32_t(wm);
-    half8_t af[4][RT];
+    half8_t af[AD][RT];
+    // A fragment is the lane's 16 bytes at a scalar offset (row tile and K32
+    // step); a row tile past the padded rows takes an out-of-range lane offset
+    // at scalar offset 0 instead.
+    const uint32_t tiles16 = (a.M + 15) / 16;
     auto load_a = [&](half8_t (&dst)[RT], uint32_t kb32) {
 #pragma unroll
-        for (int i = 0; i < RT; ++i)
+        for (int i = 0; i < RT; ++i) {
+            const bool live = RT == 1 || rb0 + WM * i < tiles16;   // uniform
+            if constexpr (RT == 1) {   // one tile: the whole offset in the lane's (range-checked)
+                dst[0] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                         arsrc, uint32_t(afrag_offset(rb0, kb0 + kb32, I, lane)), 0, 0));
+                continue;
+            }
+            const uint32_t at = live ? uint32_t(afrag_offset(rb0 + WM * i, kb0 + kb32, I, 0)) : 0u;
             dst[i] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                                     arsrc, uint32_t(afrag_offset(rb0 + WM * i, kb0 + kb32, I, lane)), 0, 0));
+                                                     arsrc, uint32_t(lane) * 16u | (live ? 0u : 0x80000000u), at, 0));
+        }
     };
     float4_t acc[RT][CT];
 #pragma unroll
@@ -161,7 +177,7 @@ __global__ __launch_bounds__(256) void gemm_narrow_kernel(const uint32_t* trelli
 #pragma unroll
     for (int d = 0; d < D; ++d) load_stage(ring[d], d);
 #pragma unroll
-    for (int k32 = 0; k32 < 4; ++k32) load_a(af[k32], k32);
+    for (int k32 = 0; k32 < AD; ++k32) load_a(af[k32], k32);
     decode_stage(ring[0], 0);
     load_stage(ring[0], D);
     __syncthreads();
@@ -182,8 +198,9 @@ __global__ __launch_bounds__(256) void gemm_narrow_kernel(const uint32_t* trelli
                 for (int i = 0; i < RT; ++i)
 #pragma unroll
                     for (int j = 0; j < CT; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[k32][i], bf[j], acc[i][j], 0, 0, 0);
-                if (st + 1 < stages) load_a(af[k32], (st + 1) * 4 + k32);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[k32 % AD][i], bf[j], acc[i][j], 0, 0, 0);
+                if (k32 + AD < 4 || st + 1 < stages) load_a(af[k32 % AD], st * 4 + k32 + AD);
+                if constexpr (RT >= 4) __builtin_amdgcn_sched_barrier(0);   // bounds the live fragments
             }
             if (st + 1 >= stages) break;
             const int slot = (d + 1) % D;   // compile-time after unrolling

@@ -168,9 +168,10 @@ uint32_t narrow_splits(const DeviceWeights& w) {
 
 // Rows per workgroup of the narrow core: the fewest that hold the pass, so that
 // no row tile multiplies padding, up to 128; 256 halves the decode per row, but
-// only two such workgroups fit a CU, so it is taken where they fill the 256 CUs
-// at that (measured at 200 rows, 128 -> 256: 4096 -> 12288 46.2 -> 43.5, 1280 ->
-// 32768 42.3 -> 37.8, 5120^2 32.4 -> 32.8, 5120 -> 1152 20.7 -> 22.0 us).
+// three such workgroups fill a CU where four or five of the others do, so it is
+// taken where two per CU exist (measured at 200 rows, 128 -> 256: 4096 -> 12288
+// 44.6 -> 41.2, 1280 -> 32768 40.1 -> 37.1, 5120^2 30.7 -> 29.3, 5120 -> 1152 20.9 ->
+// 22.4 us).
 uint32_t narrow_rows(uint64_t m, const DeviceWeights& w) {
     if (m <= 128) return m <= 16 ? 16 : m <= 32 ? 32 : m <= 64 ? 64 : 128;
     return uint64_t(w.output / 64) * narrow_splits(w) * ((m + 255) / 256) >= 512 ? 256 : 128;
