@@ -115,8 +115,7 @@ static GemvLaunch make_launch(const DeviceWeights& w, const GroupWeights* table,
     a.ncg = w.output / 128;
     a.groups = groups;
     l.rows_template = rows_template(call.rows);
-    // Split-major 1-D grid (gemv_slot).
-    l.grid = dim3(a.ncg * groups * sh.splits, 1, 1);
+    l.grid = dim3(a.ncg, groups, sh.splits);   // split-major (gemv_slot)
     l.codebook = w.codebook;
     l.lds = size_t(l.rows_template) * (32u * sh.bps + 2048u);
     l.stream = stream;
@@ -124,7 +123,7 @@ static GemvLaunch make_launch(const DeviceWeights& w, const GroupWeights* table,
 }
 
 // The per-split buffer resource spans bps rows of tiles and must stay below
-// 2^31 bytes (its out-of-range sentinel); the 1-D grid holds every column
+// 2^31 bytes (its out-of-range sentinel); the grid holds every column
 // group x split; the planes of one column group fit a buffer resource.
 static bool gemv_fits(const DeviceWeights& w, uint32_t groups, uint64_t rows) {
     const GemvShape sh = gemv_shape(w.input, w.output, w.bits);

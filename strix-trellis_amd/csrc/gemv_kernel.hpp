@@ -4,7 +4,7 @@
 // Replaces the reference's generic GEMV family (src/gemv_lds.hip:14-168,
 // src/gemv_fused.hip:17-128, src/transforms.hpp:8-52) with one wave64 design:
 //
-//   1-D grid of 256-thread workgroups (4 waves).  Workgroup (c, s, z) owns
+//   Grid of 256-thread workgroups (4 waves).  Workgroup (c, z, s) owns
 //   output columns [128c, 128c+128) of group z and input blocks
 //   [s*bps, (s+1)*bps) (16 channels each, bps a multiple of 8 so the split
 //   holds whole H128 input blocks).  The grid runs split-major: every column
@@ -61,22 +61,17 @@ __device__ __forceinline__ GroupWeights group_weights(const GemvArgs& a, int z) 
     return a.table ? a.table[z] : a.w;
 }
 
-// Workgroup L -> column group cz = L % (groups * ncg) (cz = z * ncg + c) and
-// split s = L / (groups * ncg).  The grid holds exactly groups * ncg * S
-// workgroups.  (A layout that also kept a column group's splits on one XCD --
-// workgroup L runs on XCD L % 8 -- measured slower: the device-scope partials
-// are written through to memory either way.)
+// Grid (N / 128, groups, splits): column group c of group z, split s, dispatched
+// split-major (x fastest).  A one-dimensional grid took two integer divisions
+// ahead of every workgroup's first load (4096^2 K4 R1 6.44 -> 6.35 us, 16 x 4096 -> 1024
+// K5 R4 17.30 -> 16.89).  (A layout that also kept a column
+// group's splits on one XCD -- workgroup L runs on XCD L % 8 -- measured slower:
+// the device-scope partials are written through to memory either way.)
 struct GemvSlot {
     uint32_t c, s, z, cz;
 };
 __device__ __forceinline__ GemvSlot gemv_slot(const GemvArgs& a) {
-    const uint32_t cgs = a.ncg * a.groups, L = blockIdx.x;
-    GemvSlot r;
-    r.s = L / cgs;
-    r.cz = L - r.s * cgs;
-    r.z = r.cz / a.ncg;
-    r.c = r.cz - r.z * a.ncg;
-    return r;
+    return {blockIdx.x, blockIdx.z, blockIdx.y, blockIdx.y * a.ncg + blockIdx.x};
 }
 
 // Output-stage operands of one lane's two columns (128c + lane, +64), loaded
@@ -104,9 +99,8 @@ __device__ __forceinline__ ColumnOperands column_operands(const GroupWeights& gw
     return o;
 }
 
-// Output stage of column group c for every row: fold, H32, epilogue.  Rows
-// are spread over the waves of the grid's y dimension (one row per wave and
-// step; a grid with gridDim.y == 1 walks all rows in its four waves).
+// Output stage of column group c for every row: fold, H32, epilogue, one row
+// per wave and step.
 // `plane(s, r)` returns the pointer to the 128 values of split s, row r.
 // The splits are folded in ascending order from +0; all their loads are
 // issued before the first add (one memory round trip per kFoldBatch splits).
@@ -114,7 +108,7 @@ template <typename Plane>
 __device__ __forceinline__ void finish_columns(const GemvArgs& a, const GroupWeights& gw, const ColumnOperands& op,
                                                float* y, int c, int splits, Plane plane) {
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (uint32_t r = blockIdx.y * GEMV_WAVES + w; r < a.rows; r += gridDim.y * GEMV_WAVES) {
+    for (uint32_t r = w; r < a.rows; r += GEMV_WAVES) {
         float z0 = 0.0f, z1 = 0.0f;
         for (int s = 0; s < splits; s += kFoldBatch) {
             float v0[kFoldBatch], v1[kFoldBatch];
@@ -789,7 +783,7 @@ void gemv_kernel(const uint32_t* trellis, const uint16_t* suh, const float* x0, 
     Chunk<K> ring[kGemvRing];
     load_chunk(ring[0], rsrc, block_off(0));
     __builtin_amdgcn_sched_barrier(0);
-    if (blockIdx.x < first_round_end) {
+    if (uint32_t(s) * (a.ncg * a.groups) + place.cz < first_round_end) {
         // every load but block 0's (one instruction for K <= 4, two above)
         if constexpr (K <= 4) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
         else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
@@ -1094,7 +1088,7 @@ hipError_t decode_dispatch(uint32_t codebook, const uint32_t* trellis, uint32_t 
             a.rows > 0xFFu || a.mode > 0xFFu || a.x_row_stride > 0xFFFFFFFFull)                           \
             return hipErrorInvalidValue;                                                                  \
         /* two dispatch rounds (257..512 workgroups): the first round ends at grid - 256 */               \
-        const uint32_t gx = l.grid.x;                                                                     \
+        const uint32_t gx = l.grid.x * l.grid.y * l.grid.z;                                               \
         const uint32_t fre = gx > kGemvCus && gx <= 2 * kGemvCus ? gx - kGemvCus : 0u;                    \
         hipLaunchKernelGGL(table[l.codebook][ri], l.grid, dim3(GEMV_THREADS), l.lds, l.stream, a.w.trellis, \
                            a.w.suh, a.x, a.state.epochs, a.table, a.ncg | (a.groups << 16),                \
