@@ -34,35 +34,6 @@ __device__ __forceinline__ float half_bits_to_float(uint16_t bits) {
     return (float)__builtin_bit_cast(_Float16, bits);
 }
 
-// v of lane l ^ S, without the LDS crossbar: DPP quad permutes for strides 1
-// and 2, two bank-masked row shifts for 4, a row rotate for 8, and the gfx950
-// permlane swaps (odd/even 16-lane rows, upper/lower 32-lane halves) for 16
-// and 32.
-template <int S>
-__device__ __forceinline__ float xor_lane(float v) {
-    const int lane = threadIdx.x & 63;
-    const int iv = __builtin_bit_cast(int, v);
-    if constexpr (S == 1) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0xB1, 0xf, 0xf, false));   // quad_perm 1,0,3,2
-    } else if constexpr (S == 2) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0x4E, 0xf, 0xf, false));   // quad_perm 2,3,0,1
-    } else if constexpr (S == 4) {
-        // Banks 0 and 2 of each row (lanes 0-3, 8-11) take lane + 4 (row_shl:4),
-        // banks 1 and 3 take lane - 4 (row_shr:4) over that result.
-        const int up = __builtin_amdgcn_update_dpp(iv, iv, 0x104, 0xf, 0x5, false);
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, iv, 0x114, 0xf, 0xA, false));
-    } else if constexpr (S == 8) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0x128, 0xf, 0xf, false));  // row_ror:8
-    } else if constexpr (S == 16) {
-        const auto r = __builtin_amdgcn_permlane16_swap(uint32_t(iv), uint32_t(iv), false, false);
-        return __builtin_bit_cast(float, (lane & 16) ? r[0] : r[1]);
-    } else {
-        static_assert(S == 32, "lane exchange stride");
-        const auto r = __builtin_amdgcn_permlane32_swap(uint32_t(iv), uint32_t(iv), false, false);
-        return __builtin_bit_cast(float, (lane & 32) ? r[0] : r[1]);
-    }
-}
-
 // +1 on lanes with bit S clear, -1 where it is set.
 template <int S>
 __device__ __forceinline__ float lane_sign() {
@@ -70,13 +41,32 @@ __device__ __forceinline__ float lane_sign() {
 }
 
 // One butterfly level at DPP stride S (1, 2, 4, 8) on a lane's value: the
-// lower lane keeps own + partner, the upper one partner - own.  Both are
-// fma(sign, own, partner): sign * own is exact (a sign flip), so the fma
-// rounds once, to the same bits as the add or subtract, signed zeros
-// included (a NaN operand gives a NaN either way).
+// lower lane keeps own + partner, the upper one partner - own, both as
+// partner + sign * own (the product is exact, so one rounding, signed zeros
+// included; a NaN operand gives a NaN either way).  The partner comes through
+// the add's own DPP operand: quad permutes for strides 1 and 2, a row rotate
+// for 8, and for 4 two adds, banks 0 and 2 of each row (lanes 0-3, 8-11) taking
+// lane + 4 and banks 1 and 3 lane - 4.  (A DPP move and an fma per level took
+// 8.3 cycles for 6.5, and 15 for 10.7 at stride 4.)
 template <int S>
 __device__ __forceinline__ float bfly_lane(float v, float sign) {
-    return __builtin_fmaf(sign, v, xor_lane<S>(v));
+    static_assert(S == 1 || S == 2 || S == 4 || S == 8, "DPP stride");
+    const float t = sign * v;
+    if constexpr (S == 4) {
+        // The DPP operand needs two wait states after a write of v, which the
+        // compiler does not know of an asm statement.
+        float d;
+        asm("s_nop 1\n\t"
+            "v_add_f32_dpp %0, %1, %2 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+            "v_add_f32_dpp %0, %1, %2 row_shr:4 row_mask:0xf bank_mask:0xa"
+            : "=&v"(d)
+            : "v"(v), "v"(t));
+        return d;
+    } else {
+        constexpr int ctrl = S == 1 ? 0xB1 : S == 2 ? 0x4E : 0x128;   // quad_perm 1,0,3,2 / 2,3,0,1, row_ror:8
+        const int iv = __builtin_bit_cast(int, v);
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, iv, ctrl, 0xf, 0xf, true)) + t;
+    }
 }
 
 // The level at stride 16 or 32 on the lane's two values at once: one swap
