@@ -35,26 +35,29 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_finish_kernel(GemvArgs a) {
 }
 
 // Fold of the prefill GEMM's K-split planes [S][rows][N] (written by the
-// previous launch) and the output stage: grid (N/128, ceil(rows/16)), each
-// wave four rows.  Per batch of four splits the wave issues all 32 plane loads
-// before the first add, and the four rows' H32 butterflies are interleaved;
-// every row is still folded from +0 in ascending split order, so its bits are
-// those of the one-row-per-wave fold.
-constexpr uint32_t kPlaneRowsPerWave = 4;
+// previous launch) and the output stage: grid (N/128, ceil(rows / (4 P))), each
+// wave P rows.  Per batch of SB splits the wave issues all 2 P SB plane loads
+// before the first add, and the P rows' H32 butterflies are interleaved; every
+// row is still folded from +0 in ascending split order, so its bits are those of
+// the one-row-per-wave fold.  Four rows and four splits where the rows fill the
+// chip (the fold is then bound by the planes' bytes); two rows and eight splits
+// below 512 such workgroups, where it is bound by round trips: twice the waves,
+// and up to eight splits in one (calls of 5120^2 K5 at 64 rows 22.0 -> 20.5, 5120 -> 1280
+// K4 at 128 rows 17.9 -> 16.1 us).
+template <int P, int SB>
 __global__ __launch_bounds__(GEMV_THREADS) void plane_finish_kernel(GemvArgs a) {
     const int c = blockIdx.x, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const uint32_t r0 = (blockIdx.y * GEMV_WAVES + w) * kPlaneRowsPerWave;
+    const uint32_t r0 = (blockIdx.y * GEMV_WAVES + w) * P;
     if (r0 >= a.rows) return;
     const ColumnOperands op = column_operands(a.w, c, a.N);
-    constexpr int P = int(kPlaneRowsPerWave);
     float z0[P], z1[P];
 #pragma unroll
     for (int i = 0; i < P; ++i) z0[i] = z1[i] = 0.0f;
     const float* base = a.partials + 128 * c + lane;
-    for (uint32_t s = 0; s < a.splits; s += 4) {
-        float v0[4][P], v1[4][P];
+    for (uint32_t s = 0; s < a.splits; s += SB) {
+        float v0[SB][P], v1[SB][P];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < SB; ++u)
 #pragma unroll
             for (int i = 0; i < P; ++i) {
                 // Past the last split or row: a valid address again, unused.
@@ -65,7 +68,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void plane_finish_kernel(GemvArgs a) 
                 v1[u][i] = p[64];
             }
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < SB; ++u)
             if (s + u < a.splits)
 #pragma unroll
                 for (int i = 0; i < P; ++i) {
@@ -156,9 +159,14 @@ hipError_t launch_plane_finish(const DeviceWeights& w, const LinearCall& call, c
     a.splits = splits;
     a.alpha = call.alpha;
     a.beta = call.beta;
-    constexpr uint64_t rows_per_wg = GEMV_WAVES * kPlaneRowsPerWave;
-    const uint32_t row_groups = uint32_t((call.rows + rows_per_wg - 1) / rows_per_wg);
-    hipLaunchKernelGGL(plane_finish_kernel, dim3(w.output / 128, row_groups, 1), dim3(GEMV_THREADS), 0, stream, a);
+    auto grid = [&](uint32_t rows_per_wave) {
+        const uint64_t rows = GEMV_WAVES * uint64_t(rows_per_wave);
+        return dim3(w.output / 128, uint32_t((call.rows + rows - 1) / rows), 1);
+    };
+    if (uint64_t(grid(4).x) * grid(4).y >= 512)
+        hipLaunchKernelGGL((plane_finish_kernel<4, 4>), grid(4), dim3(GEMV_THREADS), 0, stream, a);
+    else
+        hipLaunchKernelGGL((plane_finish_kernel<2, 8>), grid(2), dim3(GEMV_THREADS), 0, stream, a);
     return hipGetLastError();
 }
 
