@@ -117,10 +117,15 @@ __device__ __forceinline__ void link_chunk(Chunk<K>& c, bool first_of_tile) {
 // ---------------------------------------------------------------------------
 // Window of the state at chunk position (V, F): fragment lane 4g+V, fragment F.
 // Its 16 bits end (8V+F+1)*K bits after the chunk start; state() returns them
-// zero-extended.  Two windows 16 bits apart share one v_alignbit (K = 1, 2, 4,
-// 8): the lower is its low half (v_and), the upper its high half (v_lshrrev).
-// Other widths have no such pairs: a window inside one word is one v_bfe, one
-// that crosses words a v_alignbit and a v_and.
+// zero-extended.  With r the window's distance from the low end of its word:
+//   r = 0, 16       the word's low or high half (v_and, v_lshrrev);
+//   0 < r < 16      inside the word: one v_bfe;
+//   r > 16          crosses into the next word: one v_alignbit per word boundary,
+//                   at the lowest such r, holds every window that crosses there
+//                   (they start at most 14 bits later), each a v_and or a v_bfe.
+// (Against one v_alignbit per crossing window, or per pair of windows 16 bits
+// apart: routed experts 4096 <-> 1536 K2, 8 tokens, 122.7 -> 115.0 us; output head
+// 5120 -> 129280 K6 100.2 -> 97.3; GEMV of 4096 -> 12288 1-6 %.)
 // ---------------------------------------------------------------------------
 template <int K, int V, int F>
 struct Window {
@@ -128,16 +133,13 @@ struct Window {
     static constexpr int shift = 32 * K - end;   // distance of the window LSB from the chunk LSB
     static constexpr int q = shift / 32;
     static constexpr int r = shift % 32;
-    static constexpr bool paired = 16 % K == 0;
-    static constexpr bool hi = r == 16 || (r > 16 && paired);
-    static constexpr int align = hi ? r - 16 : r;
+    static constexpr int anchor = r > 16 ? r - (r - 17) / K * K : 0;   // lowest window start above 16 in the word
 
     __device__ __forceinline__ static uint32_t state(const Chunk<K>& c) {
-        uint32_t w;
-        if constexpr (align == 0) w = c.template lsb<q>();
-        else if constexpr (!paired && r < 16) return (c.template lsb<q>() >> r) & 0xFFFFu;
-        else w = __builtin_amdgcn_alignbit(c.template lsb<q + 1>(), c.template lsb<q>(), align);
-        return hi ? w >> 16 : w & 0xFFFFu;
+        const uint32_t w = c.template lsb<q>();
+        if constexpr (r == 16) return w >> 16;
+        else if constexpr (r < 16) return (w >> r) & 0xFFFFu;
+        else return (__builtin_amdgcn_alignbit(c.template lsb<q + 1>(), w, anchor) >> (r - anchor)) & 0xFFFFu;
     }
 };
 
