@@ -20,7 +20,7 @@
 //     lane and fragment.  WM balances the two sources: more waves along M read
 //     fewer A fragments twice and more B ones;
 //   * raw core rows go to planes[split][M][N] whatever the split count; with row
-//     blocks of 16 or 32 the last workgroup of a 128-column group folds them and
+//     blocks of 16 the last workgroup of a 128-column group folds them and
 //     applies the output stage itself, otherwise a second launch does
 //     (plane_finish_kernel).
 // Per-output accumulation: MFMA K32 steps in ascending K from +0 (the order
@@ -30,8 +30,8 @@
 // Measured against 128 x 128 and 256 x 128 tiles of the same order (64 KiB of
 // LDS, two waves along each dimension; 320 workgroups on 5120^2 that multiplied
 // 128 rows whatever M was), calls, same bits: 5120^2 K5 M = 16 / 24 / 64 / 128 /
-// 200 24.5 / 24.6 / 27.6 / 30.9 / 40.7 -> 14.4 / 16.7 / 21.3 / 24.5 / 29.2 us, 4096
-// -> 12288 K6 29.1 / 29.4 / 32.0 / 35.7 / 49.7 -> 17.8 / 19.7 / 23.5 / 30.2 / 40.8 us,
+// 200 24.5 / 24.6 / 27.6 / 30.9 / 40.7 -> 14.3 / 15.8 / 19.8 / 24.4 / 29.2 us, 4096
+// -> 12288 K6 29.1 / 29.4 / 32.0 / 35.7 / 49.7 -> 17.9 / 19.0 / 23.5 / 30.2 / 40.8 us,
 // 1152 -> 5120 K4 M = 16 / 128 25.0 / 30.3 -> 11.9 / 16.7 us; 5120 -> 1152 K4 M =
 // 512 / 4096 31.5 / 143.9 -> 27.0 / 127.9 us.
 //
@@ -308,14 +308,14 @@ struct GemmLaunch {
 template <int K>
 hipError_t gemm_narrow_dispatch(const GemmLaunch& l);
 
-// Row tiles of 16 per workgroup: 1, 2 or 4 with the fold, 8 or 16 without.
+// Row tiles of 16 per workgroup: 1 with the fold, 2, 4, 8 or 16 without.
 #define STX_INSTANTIATE_GEMM_NARROW(K)                                                                          \
     template <>                                                                                                \
     hipError_t gemm_narrow_dispatch<K>(const GemmLaunch& l) {                                                   \
         using Fn = void (*)(const uint32_t*, const _Float16*, uint32_t, uint32_t, uint32_t, uint32_t, GemmArgs); \
         static const Fn table[5][3] = {                                                                        \
             {gemm_narrow_kernel<K, 0, 1, true>, gemm_narrow_kernel<K, 1, 1, true>, gemm_narrow_kernel<K, 2, 1, true>}, \
-            {gemm_narrow_kernel<K, 0, 2, true>, gemm_narrow_kernel<K, 1, 2, true>, gemm_narrow_kernel<K, 2, 2, true>}, \
+            {gemm_narrow_kernel<K, 0, 2, false>, gemm_narrow_kernel<K, 1, 2, false>, gemm_narrow_kernel<K, 2, 2, false>}, \
             {gemm_narrow_kernel<K, 0, 4, false>, gemm_narrow_kernel<K, 1, 4, false>, gemm_narrow_kernel<K, 2, 4, false>}, \
             {gemm_narrow_kernel<K, 0, 8, false>, gemm_narrow_kernel<K, 1, 8, false>, gemm_narrow_kernel<K, 2, 8, false>}, \
             {gemm_narrow_kernel<K, 0, 16, false>, gemm_narrow_kernel<K, 1, 16, false>, gemm_narrow_kernel<K, 2, 16, false>}}; \

@@ -172,18 +172,21 @@ uint32_t narrow_splits(const DeviceWeights& w) {
 // taken where two per CU exist (measured at 200 rows, 128 -> 256: 4096 -> 12288
 // 44.6 -> 41.2, 1280 -> 32768 40.1 -> 37.1, 5120^2 30.7 -> 29.3, 5120 -> 1152 20.9 ->
 // 22.4 us).
+// Blocks of 16 rows fold their planes in the last workgroup (narrow_counters),
+// which with 16 splits takes longer than 32-row blocks and a folding launch
+// (2048^2 K4 at 16 rows 14.4 -> 11.6 us).
 uint32_t narrow_rows(uint64_t m, const DeviceWeights& w) {
-    if (m <= 128) return m <= 16 ? 16 : m <= 32 ? 32 : m <= 64 ? 64 : 128;
+    if (m <= 128) return m <= 16 && narrow_splits(w) <= 8 ? 16 : m <= 32 ? 32 : m <= 64 ? 64 : 128;
     return uint64_t(w.output / 64) * narrow_splits(w) * ((m + 255) / 256) >= 512 ? 256 : 128;
 }
 
 // Arrival counters (one per 128-column group and row block) of a narrow pass
 // whose workgroups fold the planes themselves, else 0.  The last arrival folds
-// a row block alone, which beats a launch of its own for up to 32 rows (5120^2
-// K5 M = 16 / 32: 17.0 / 18.3 -> 14.2 / 16.8 us) and loses from 64 on (22.2 -> 24.5).
+// a row block alone, which beats a launch of its own for up to 16 rows (5120^2
+// K5: 17.0 -> 14.2 us) and loses from 17 on (5120^2 K5 / 5120 -> 1280 K4 at 24 rows
+// 16.4 / 13.5 in the last workgroup, 15.8 and 11.7 in a launch).
 uint32_t narrow_counters(uint64_t m, const DeviceWeights& w) {
-    const uint32_t r = narrow_rows(m, w);
-    return !gemm_wide(m, w) && r <= 32 ? uint32_t((m + r - 1) / r) * (w.output / 128) : 0;
+    return !gemm_wide(m, w) && narrow_rows(m, w) == 16 ? w.output / 128 : 0;
 }
 
 // Whether a launch of its own folds the pass's planes.

@@ -2,8 +2,8 @@
 
 Every call of fewer than 256 rows, and any call on a layer whose width is not a
 multiple of 256, runs workgroups of 16, 32, 64, 128 or 256 rows; blocks of 16
-and 32 rows fold their K-split planes in the last workgroup to arrive, the
-others in a second launch.  Checked here on both sides of every block size:
+rows fold their K-split planes in the last workgroup to arrive, the others in a
+second launch.  Checked here on both sides of every block size:
   * the full operator against the oracle's staged FP32 layer (reference GPU
     gate, docs/GPU_TESTS.md:124-143) on the first and last rows;
   * every row's bits equal those of the same row in the largest call (one
