@@ -354,7 +354,8 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
     // ones back: 2,940 cycles per stage for 2,048 of MFMA.  Measured against
     // that loop, same bits: M = 512 on 5120^2 59.5 -> 57.0 us, M = 2048 on 4096
     // -> 12288 225.2 -> 221.1 us, M = 3000 on 1280 -> 16384 173.4 -> 167.5 us.
-    // M takes 1,080-1,130 cycles (1,024 of MFMA), D about 1,550: D bounds the slot.
+    // With marks that pin the phases: M 1,111 cycles (1,024 of MFMA), D 1,295, 260 and
+    // 239 at their barriers, 2,905 per stage.
     //
     // D(n) decodes the half's two blocks of stage n into B buffer n % 2, DMAs
     // its half of the core input of stage n + 1 into A buffer (n + 1) % 3,
