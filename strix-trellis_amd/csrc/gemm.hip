@@ -76,10 +76,9 @@ extern "C" int strix_amd_debug_stage_clock(void* records) {
 
 hipError_t launch_gemm(const DeviceWeights& w, const LinearCall& call, hipStream_t stream) {
     if (uint64_t(w.input / 16) * (w.output / 16) * 32u * w.bits >= (uint64_t(1) << 31)) return hipErrorInvalidValue;
-    const uint64_t pass = gemm_pass_rows(w);
     _Float16* afrag = static_cast<_Float16*>(call.workspace);
-    for (uint64_t r0 = 0; r0 < call.rows; r0 += pass) {
-        const uint64_t m = call.rows - r0 < pass ? call.rows - r0 : pass;
+    for (uint64_t r0 = 0, m; r0 < call.rows; r0 += m) {
+        m = gemm_next_pass(w, call.rows - r0);
         // 256 x 256 tiles (32x16 fragments) once the rows fill them and N splits
         // into 256-column blocks; the narrow core (16x32 fragments) otherwise.
         const bool wide = gemm_wide(m, w);

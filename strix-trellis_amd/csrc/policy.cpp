@@ -224,30 +224,56 @@ uint64_t pass_workspace(const DeviceWeights& w, uint64_t m) {
            (s > 1 ? align256(uint64_t(s) * m * w.output * sizeof(float)) : 0);
 }
 
+// Rows of the next pass of a call that has `rows` left.  A narrow pass writes
+// narrow_splits planes of M x N floats (as large as its output where one split
+// suffices), so its rows are also bounded by kPassPlaneBytes; at least one
+// 16-row tile.  Every row of every narrow pass has the same bits, so cutting a
+// call does not show in its results.
+uint64_t gemm_next_pass(const DeviceWeights& w, uint64_t rows) {
+    const uint64_t pass = gemm_pass_rows(w), m = rows < pass ? rows : pass;
+    if (gemm_wide(m, w)) return m;
+    uint64_t cap = kPassPlaneBytes / (uint64_t(narrow_splits(w)) * w.output * sizeof(float));
+    cap -= cap % (cap >= 256 ? 256 : 16);
+    if (cap < 16) cap = 16;
+    return m < cap ? m : cap;
+}
+
+// Calls visit(rows of a pass, passes of that size) for the passes of a call:
+// whole ones, then what is left (a wide layer's remainder may be narrow, and
+// then be cut again).
+template <class Visit>
+static void gemm_passes(const DeviceWeights& w, uint64_t rows, Visit visit) {
+    while (rows) {
+        const uint64_t m = gemm_next_pass(w, rows);
+        visit(m, rows / m);
+        rows %= m;
+    }
+}
+
 uint64_t gemm_workspace_bytes(const DeviceWeights& w, uint64_t rows) {
-    const uint64_t pass = gemm_pass_rows(w);
-    if (rows <= pass) return pass_workspace(w, rows);
-    const uint64_t a = pass_workspace(w, pass), b = rows % pass ? pass_workspace(w, rows % pass) : 0;
-    return a > b ? a : b;
+    uint64_t bytes = 0;
+    gemm_passes(w, rows, [&](uint64_t m, uint64_t) {
+        const uint64_t b = pass_workspace(w, m);
+        if (b > bytes) bytes = b;
+    });
+    return bytes;
 }
 
 uint32_t gemm_launch_count(const DeviceWeights& w, uint64_t rows) {
-    const uint64_t pass = gemm_pass_rows(w);
-    uint32_t n = 0;
-    for (uint64_t r0 = 0; r0 < rows; r0 += pass) {
-        const uint64_t m = rows - r0 < pass ? rows - r0 : pass;
-        n += 2;
-        n += pass_folds(m, w);
+    uint64_t n = 0;
+    gemm_passes(w, rows, [&](uint64_t m, uint64_t passes) {
+        uint32_t per = 2 + pass_folds(m, w);
         if (gemm_wide(m, w)) {
             const WideSplit sp = wide_split(m, w);
-            n += sp.full && sp.half;
+            per += sp.full && sp.half;
         }
-    }
-    return n;
+        n += passes * per;
+    });
+    return uint32_t(n);
 }
 
 uint32_t gemm_split_count(const DeviceWeights& w, uint64_t rows) {
-    const uint64_t pass = gemm_pass_rows(w), m = rows < pass ? rows : pass;
+    const uint64_t m = gemm_next_pass(w, rows);
     return gemm_wide(m, w) ? wide_splits(m, w) : narrow_splits(w);
 }
 

@@ -17,7 +17,9 @@ struct Handoff {
     uint32_t q = 0, x = 0;
 };
 constexpr uint32_t kWideSplitMinStages = 8;   // 64-channel stages per K split, at least
+constexpr uint64_t kPassPlaneBytes = uint64_t(1) << 30;   // planes of one narrow pass, at most
 uint64_t gemm_pass_rows(const DeviceWeights& w);
+uint64_t gemm_next_pass(const DeviceWeights& w, uint64_t rows);
 uint64_t afrag_bytes(const DeviceWeights& w, uint64_t m);
 bool wide_can_split(const DeviceWeights& w);
 WideSplit wide_split(uint64_t m, const DeviceWeights& w);

@@ -867,6 +867,42 @@ static void policy_rules() {
     CHECK(stx::moe_split_staged(1152).bps == 18 && stx::moe_down_groups(18, 1) == 3 && stx::moe_down_groups(18, 3) == 3);
 }
 
+// Passes of a GEMM call: they cover its rows, each fits the call's workspace and
+// is counted, and what the library asks for beside the fragments of one pass
+// stays bounded however many rows the call has (a narrow layer's planes are
+// cut to kPassPlaneBytes, or to one 16-row tile where even that is larger).
+static void pass_rules() {
+    for (uint32_t I : {128u, 384u, 1152u, 4096u})
+        for (uint32_t N : {128u, 384u, 1152u, 8320u, 12288u, 32896u, (1u << 22) - 256u, (1u << 22) + 128u}) {
+            stx::DeviceWeights w;
+            w.input = I;
+            w.output = N;
+            w.bits = 1;
+            const uint64_t tile = uint64_t(stx::narrow_splits(w)) * 16 * N * 4;
+            const uint64_t most = tile > stx::kPassPlaneBytes ? tile : stx::kPassPlaneBytes;
+            for (uint64_t rows : {1ull, 16ull, 17ull, 255ull, 256ull, 511ull, 3000ull, 8191ull, 70001ull, 5000000ull}) {
+                const uint64_t ws = stx::gemm_workspace_bytes(w, rows);
+                uint64_t left = rows, launches = 0;
+                while (left) {
+                    const uint64_t m = stx::gemm_next_pass(w, left);
+                    CHECK(m >= 1 && m <= left && m <= stx::gemm_pass_rows(w));
+                    CHECK(stx::pass_workspace(w, m) <= ws);
+                    launches += 2 + stx::pass_folds(m, w);
+                    if (stx::gemm_wide(m, w)) {
+                        const stx::WideSplit sp = stx::wide_split(m, w);
+                        launches += sp.full && sp.half;
+                    } else {
+                        CHECK(uint64_t(stx::narrow_splits(w)) * m * N * 4 <= most);
+                        CHECK(m == left || m % 16 == 0);   // whole row tiles but for the last pass
+                    }
+                    left -= m;
+                }
+                CHECK(stx::gemm_launch_count(w, rows) == launches);
+                if (N % 256) CHECK(ws <= stx::afrag_bytes(w, stx::gemm_pass_rows(w)) + most + N + 512);
+            }
+        }
+}
+
 // Allocation-free GEMV: no allocation, free, copy or synchronisation; the
 // planes go to the device's static scratch; the workspace fields must be
 // empty; more than 8 rows and planes beyond the scratch are rejected.
@@ -968,6 +1004,7 @@ static void stream_read_calls(strix_context c, hipStream_t hs) {
 
 int main() {
     policy_rules();
+    pass_rules();
     context_rules();
     strix_context_desc cd = header<strix_context_desc>();
     strix_context c = nullptr;

@@ -71,3 +71,23 @@ def test_narrow_row_blocks(ctx, I, N, K, codebook, splits):
         want = linear.apply_alpha_beta(y.cpu().numpy(), old.cpu().numpy(), -0.5, 2.0)
         np.testing.assert_array_equal(y_ab.cpu().numpy().view(np.uint32), want.view(np.uint32))
     w.destroy()
+
+
+def test_narrow_passes(ctx):
+    """A call whose planes pass 1 GiB runs in several passes, each row with the
+    bits of a call of its own rows."""
+    I, N, K, M = 128, 32896, 2, 8200
+    print(f"narrow gemm passes {I}x{N} K={K} M={M}", flush=True)
+    tr, suh, svh, b = synth.layer(I, N, K, 7300, bias=True)
+    w = runtime.Weights(ctx, tr, suh, svh, b, "mul1")
+    x = torch.from_numpy(synth.activations(M, I, 7301)).to(DEV)
+    y = torch.full((M, N), float("nan"), device=DEV)
+    ws = runtime.workspace_bytes(w, x, y)
+    assert ws < (1 << 30) + M * I * 2 + (1 << 20) < M * N * 4 + M * I * 2
+    runtime.gemm(w, x, y)
+    edge = (1 << 30) // (N * 4) // 256 * 256   # rows of the first pass
+    for a, e in ((0, 40), (edge - 40, edge), (edge, edge + 40), (M - 40, M)):
+        part = torch.empty((e - a, N), device=DEV)
+        runtime.gemm(w, x[a:e].contiguous(), part)
+        assert torch.equal(_bits(y[a:e]), _bits(part)), (a, e)
+    w.destroy()
