@@ -126,6 +126,10 @@ hipError_t launch_gemv_owner(const DeviceWeights& geometry, const GroupWeights* 
                              hipStream_t stream);
 // The library's choice between the owner-fold and the split grouped plan.
 bool grouped_owner_preferred(const DeviceWeights& geometry, uint32_t groups, uint64_t rows);
+// The narrow GEMM core folds its planes in the last workgroup to arrive for
+// passes of one 16-row block and up to this many splits.
+constexpr uint32_t kNarrowFoldRows = 16;
+constexpr uint32_t kNarrowFoldSplits = 8;
 // Prefill path (any row count): input stage to FP16 in the workspace, then the
 // MFMA core with the fused output stage.
 hipError_t launch_gemm(const DeviceWeights& w, const LinearCall& call, hipStream_t stream);

@@ -19,8 +19,8 @@
 //     order, which the input-stage kernel wrote: one coalesced 16-byte load per
 //     lane and fragment.  WM balances the two sources: more waves along M read
 //     fewer A fragments twice and more B ones;
-//   * raw core rows go to planes[split][M][N] whatever the split count; with row
-//     blocks of 16 the last workgroup of a 128-column group folds them and
+//   * raw core rows go to planes[split][M][N] whatever the split count; in a pass
+//     of one 16-row block the last workgroup of a 128-column group folds them and
 //     applies the output stage itself, otherwise a second launch does
 //     (plane_finish_kernel).
 // Per-output accumulation: MFMA K32 steps in ascending K from +0 (the order
@@ -66,7 +66,7 @@ struct GemmArgs {
     // of K between a head and a tail workgroup, 256 q whole tiles.
     uint32_t q, x;
     float* handoff;           // [x][8 waves][128 accumulators][64 lanes]
-    uint32_t* flags;          // [x], 0 at launch; narrow kernel: arrivals per 128-column group and row block
+    uint32_t* flags;          // [x], 0 at launch; narrow kernel with the fold: arrivals per 128-column group
     uint32_t poll_limit;      // tail's polls before it takes a tile over
     // K split: `splits` workgroups per tile (narrow kernel: grid z, I/splits
     // channels each; wide kernel: grid y, stage ranges) write their raw core
@@ -237,28 +237,30 @@ void gemm_narrow_kernel(const uint32_t* trellis, const _Float16* afrag, uint32_t
         // complete (waited for, then a barrier) before the arrival; the last
         // arrival reads them with device-coherent loads issued after the counter
         // result, behind a barrier.
+        static_assert(16 * TM == kNarrowFoldRows, "the fold serves a pass of one row block");
         __builtin_amdgcn_s_waitcnt(0);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __syncthreads();
         int* last = reinterpret_cast<int*>(smem);
         const uint32_t cg = uint32_t(c) >> 1;
         if (tid == 0)
-            *last = __hip_atomic_fetch_add(a.flags + uint64_t(mb) * (N / 128) + cg, 1u, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT) == 2 * a.splits - 1;
+            *last = __hip_atomic_fetch_add(a.flags + cg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                    2 * a.splits - 1;
         __syncthreads();
         if (!*last) return;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        // Wave w folds rows w, w + 4, ... of the block, P at a time, lane l
-        // columns 2l and 2l + 1: each plane from +0 in ascending split order, then
-        // H32 and the output stage (the order and operations of plane_finish_kernel).
-        constexpr int P = 4, SB = 8;
+        // Wave w folds rows w, w + 4, ..., P at a time, lane l columns 2l and 2l + 1:
+        // each plane from +0 in ascending split order, then H32 and the output stage
+        // (the order and operations of plane_finish_kernel).  Both loops run at most
+        // once; written out, the 32 loads' resources are live together and SGPRs
+        // spill (106 for 67; 5120^2 K5 at 16 rows 13.8 -> 14.0, 4096^2 K4 11.9 -> 12.2 us).
+        constexpr int P = int(kNarrowFoldRows) / 4, SB = int(kNarrowFoldSplits);
         const uint32_t n0 = 128u * cg + 2u * uint32_t(lane);
         const uint32_t svp = ld_global(reinterpret_cast<const uint32_t*>(a.svh + n0));
         const bool has_bias = a.bias != nullptr;
         const auto rb = make_rsrc(a.bias, has_bias ? N * 4u : 0u);
         const gemv_f2_t bias = __builtin_bit_cast(gemv_f2_t, __builtin_amdgcn_raw_buffer_load_b64(rb, n0 * 4u, 0, 0));
-        const uint32_t end = (uint32_t(mb) + 1) * (16 * TM) < a.M ? (uint32_t(mb) + 1) * (16 * TM) : a.M;
-        for (uint32_t r0 = uint32_t(mb) * (16 * TM) + uint32_t(w); r0 < end; r0 += 4 * P) {
+        for (uint32_t r0 = uint32_t(w); r0 < a.M; r0 += 4 * P) {
             gemv_f2_t z[P];
 #pragma unroll
             for (int i = 0; i < P; ++i) z[i] = gemv_f2_t{0.0f, 0.0f};
@@ -270,7 +272,7 @@ void gemm_narrow_kernel(const uint32_t* trellis, const _Float16* afrag, uint32_t
                     for (int i = 0; i < P; ++i) {
                         // Past the last split or row: a valid address again, unused.
                         const uint32_t ss = s0 + u < a.splits ? s0 + u : s0;
-                        const uint32_t r = r0 + 4 * i < end ? r0 + 4 * i : r0;
+                        const uint32_t r = r0 + 4 * i < a.M ? r0 + 4 * i : r0;
                         const auto ps = make_rsrc(a.planes + (uint64_t(ss) * a.M + r) * N, N * 4u);
                         v[u][i] = poll_pair(ps, n0 * 4u, 0);
                     }
@@ -286,7 +288,7 @@ void gemm_narrow_kernel(const uint32_t* trellis, const _Float16* afrag, uint32_t
             h32_pairs<P>(z);
 #pragma unroll
             for (int i = 0; i < P; ++i) {
-                if (r0 + 4 * i >= end) break;
+                if (r0 + 4 * i >= a.M) break;
                 float* yr = a.y + uint64_t(r0 + 4 * i) * N + n0;
                 gemv_f2_t o;
                 o.x = output_value(z[i].x, uint16_t(svp), has_bias, bias.x, a.alpha, a.beta, yr);
@@ -319,6 +321,9 @@ hipError_t gemm_narrow_dispatch(const GemmLaunch& l);
             {gemm_narrow_kernel<K, 0, 4, false>, gemm_narrow_kernel<K, 1, 4, false>, gemm_narrow_kernel<K, 2, 4, false>}, \
             {gemm_narrow_kernel<K, 0, 8, false>, gemm_narrow_kernel<K, 1, 8, false>, gemm_narrow_kernel<K, 2, 8, false>}, \
             {gemm_narrow_kernel<K, 0, 16, false>, gemm_narrow_kernel<K, 1, 16, false>, gemm_narrow_kernel<K, 2, 16, false>}}; \
+        /* the fold: one row block, and planes that one round trip holds */                                    \
+        if (l.bm == 16 && (l.args.M > kNarrowFoldRows || l.args.splits > kNarrowFoldSplits))                   \
+            return hipErrorInvalidValue;                                                                       \
         const int ti = l.bm == 16 ? 0 : l.bm == 32 ? 1 : l.bm == 64 ? 2 : l.bm == 128 ? 3 : 4;                  \
         const dim3 grid(l.args.N / 64, (l.args.M + l.bm - 1) / l.bm, l.args.splits);                           \
         const GemmArgs& a = l.args;                                                                            \

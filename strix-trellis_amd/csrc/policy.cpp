@@ -176,17 +176,17 @@ uint32_t narrow_splits(const DeviceWeights& w) {
 // which with 16 splits takes longer than 32-row blocks and a folding launch
 // (2048^2 K4 at 16 rows 14.4 -> 11.6 us).
 uint32_t narrow_rows(uint64_t m, const DeviceWeights& w) {
-    if (m <= 128) return m <= 16 && narrow_splits(w) <= 8 ? 16 : m <= 32 ? 32 : m <= 64 ? 64 : 128;
+    if (m <= 128) return m <= kNarrowFoldRows && narrow_splits(w) <= kNarrowFoldSplits ? 16 : m <= 32 ? 32 : m <= 64 ? 64 : 128;
     return uint64_t(w.output / 64) * narrow_splits(w) * ((m + 255) / 256) >= 512 ? 256 : 128;
 }
 
-// Arrival counters (one per 128-column group and row block) of a narrow pass
-// whose workgroups fold the planes themselves, else 0.  The last arrival folds
-// a row block alone, which beats a launch of its own for up to 16 rows (5120^2
+// Arrival counters (one per 128-column group) of a narrow pass whose workgroups
+// fold the planes themselves, else 0.  The last arrival folds a column group
+// alone, which beats a launch of its own for up to 16 rows (5120^2
 // K5: 17.0 -> 14.2 us) and loses from 17 on (5120^2 K5 / 5120 -> 1280 K4 at 24 rows
 // 16.4 / 13.5 in the last workgroup, 15.8 and 11.7 in a launch).
 uint32_t narrow_counters(uint64_t m, const DeviceWeights& w) {
-    return !gemm_wide(m, w) && narrow_rows(m, w) == 16 ? w.output / 128 : 0;
+    return !gemm_wide(m, w) && narrow_rows(m, w) == kNarrowFoldRows ? w.output / 128 : 0;
 }
 
 // Whether a launch of its own folds the pass's planes.

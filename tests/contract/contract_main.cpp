@@ -894,6 +894,16 @@ static void pass_rules() {
                     } else {
                         CHECK(uint64_t(stx::narrow_splits(w)) * m * N * 4 <= most);
                         CHECK(m == left || m % 16 == 0);   // whole row tiles but for the last pass
+                        // The fold in the last workgroup: one row block, one
+                        // counter per column group, inside the workspace.
+                        const uint32_t counters = stx::narrow_counters(m, w);
+                        CHECK((stx::narrow_rows(m, w) == stx::kNarrowFoldRows) == (counters != 0));
+                        if (counters) {
+                            CHECK(m <= stx::kNarrowFoldRows && stx::narrow_splits(w) <= stx::kNarrowFoldSplits);
+                            CHECK(counters == N / 128);
+                            CHECK(stx::pass_workspace(w, m) >=
+                                  stx::afrag_bytes(w, m) + uint64_t(stx::narrow_splits(w)) * m * N * 4 + counters * 4);
+                        }
                     }
                     left -= m;
                 }
