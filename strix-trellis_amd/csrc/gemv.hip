@@ -181,6 +181,10 @@ hipError_t launch_gemv_grouped(const DeviceWeights& geometry, const GroupWeights
                                const LinearCall& call, uint64_t x_group_stride, uint64_t y_group_stride,
                                const FusedState* state, hipStream_t stream) {
     if (!gemv_fits(geometry, groups, call.rows)) return hipErrorInvalidValue;
+    // The activation reads two contiguous outputs; refused ahead of any launch.
+    if (call.swiglu_hidden &&
+        (groups != 2 || call.y_row_stride != geometry.output || call.swiglu_row_stride < geometry.output))
+        return hipErrorInvalidValue;
     GemvLaunch l = make_launch(geometry, table, groups, call, x_group_stride, y_group_stride,
                                static_cast<float*>(call.workspace), state, stream);
     hipError_t e = gemv_table[geometry.bits - 1](l);
@@ -191,7 +195,6 @@ hipError_t launch_gemv_grouped(const DeviceWeights& geometry, const GroupWeights
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (!call.swiglu_hidden) return hipSuccess;
-    if (groups != 2 || call.y_row_stride != geometry.output) return hipErrorInvalidValue;
     return launch_swiglu_rows(call.y, call.y + y_group_stride, call.swiglu_hidden, call.swiglu_row_stride,
                               uint32_t(call.rows), geometry.output, stream);
 }

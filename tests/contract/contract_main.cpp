@@ -1012,6 +1012,114 @@ static void stream_read_calls(strix_context c, hipStream_t hs) {
     for (void* p : {src, static_cast<void*>(sink)}) CHECK(hipFree(p) == hipSuccess);
 }
 
+// SwiGLU plans: members of one rate and codebook are one grouped launch and one
+// activation launch on scratch that the plan owns; members of different rates,
+// and plans with diagnostic buffers, launch one by one.  A creation that fails
+// at any allocation, copy, fill or synchronisation leaves no allocation behind
+// and its weights free to go; submission is quiet; a plan keeps its weights.
+static void swiglu_plan(strix_context c, hipStream_t hs) {
+    strix_stream st = stream_of(hs);
+    const size_t live00 = fake::live.size();
+    auto prepare = [&](uint64_t n, uint64_t i, uint32_t k, bool bias) {
+        const HostLinear L(n, i, k, bias);
+        const strix_exl3_parts_desc parts = L.parts();
+        strix_weights w = nullptr;
+        STATUS(strix_weights_prepare_parts(c, &parts, &st, &w), STRIX_SUCCESS);
+        return w;
+    };
+    const uint64_t I = 1024, H = 256, rows = 3, stride = H + 64;
+    auto* x = static_cast<float*>(device_alloc(rows * I * 4));
+    auto* wide = static_cast<float*>(device_alloc(rows * stride * 4));
+    auto* diag = static_cast<float*>(device_alloc(2 * rows * H * 4));
+    strix_weights gate = prepare(H, I, 4, false), up = prepare(H, I, 4, true), other = prepare(H, I, 5, false);
+    strix_weights g1 = prepare(H, 128, 4, false), u1 = prepare(H, 128, 4, false);   // one input split
+    const size_t live0 = fake::live.size();
+    auto describe = [&](strix_weights g, strix_weights u, uint64_t input) {
+        strix_tp_swiglu_desc d;
+        strix_tp_swiglu_desc_init(&d);
+        d.input = tensor(x, rows * input * 4, rows, input, 2);
+        d.gate = g;
+        d.up = u;
+        d.hidden_output = tensor(wide, rows * stride * 4, rows, H, 2);
+        d.hidden_output.strides[0] = stride;
+        return d;
+    };
+    const strix_tp_swiglu_desc d = describe(gate, up, I);
+
+    // Creation: scratch, table copy, two fills of the state, one synchronisation.
+    strix_tp_swiglu_plan p = reinterpret_cast<strix_tp_swiglu_plan>(0x1);
+    auto refused = [&](strix_status want) {
+        STATUS(strix_tp_swiglu_plan_create(c, &d, &st, &p), want);
+        CHECK(p == nullptr && fake::live.size() == live0);
+        fake::reset_failures();
+        p = reinterpret_cast<strix_tp_swiglu_plan>(0x1);
+    };
+    fake::malloc_fail_at = 0;
+    refused(STRIX_ERROR_OUT_OF_MEMORY);
+    fake::malloc_fail_at = 0;
+    fake::malloc_error = hipErrorUnknown;
+    refused(STRIX_ERROR_BACKEND);
+    fake::copy_fail_at = 0;
+    refused(STRIX_ERROR_BACKEND);
+    for (int at = 0; at < 2; ++at) {
+        const fake::Counters before = fake::n;
+        fake::launch_fail_at = at;
+        refused(STRIX_ERROR_BACKEND);
+        CHECK(fake::n.syncs == before.syncs + 1);   // drained before the free
+    }
+    fake::sync_fail_at = 0;
+    refused(STRIX_ERROR_BACKEND);
+    strix_tp_swiglu_desc bad = d;
+    bad.hidden_output.data = x;   // hidden over the input
+    bad.hidden_output.buffer_bytes = rows * I * 4;
+    STATUS(strix_tp_swiglu_plan_create(c, &bad, &st, &p), STRIX_ERROR_INVALID_ARGUMENT);
+    CHECK(p == nullptr && fake::live.size() == live0);
+
+    auto submit = [&](const strix_tp_swiglu_desc& desc, std::vector<std::string> names) {
+        strix_tp_swiglu_plan q = nullptr;
+        STATUS(strix_tp_swiglu_plan_create(c, &desc, &st, &q), STRIX_SUCCESS);
+        for (int i = 0; i < 2; ++i) {
+            fake::launches.clear();
+            const fake::Counters before = fake::n;
+            STATUS(strix_tp_swiglu_plan_submit(q), STRIX_SUCCESS);
+            check_quiet_since(before);
+            CHECK(fake::launches.size() == names.size());
+            for (size_t k = 0; k < names.size(); ++k)
+                CHECK(fake::launches[k].name == names[k] && fake::launches[k].stream == hs);
+        }
+        for (size_t at = 0; at < names.size(); ++at) {   // the first failure ends the submission
+            fake::launches.clear();
+            fake::launch_fail_at = int(at);
+            STATUS(strix_tp_swiglu_plan_submit(q), STRIX_ERROR_BACKEND);
+            CHECK(fake::launches.size() == at + 1);
+            fake::reset_failures();
+        }
+        STATUS(strix_weights_destroy(desc.gate), STRIX_ERROR_INVALID_ARGUMENT);   // the plan keeps them
+        STATUS(strix_weights_destroy(desc.up), STRIX_ERROR_INVALID_ARGUMENT);
+        STATUS(strix_tp_swiglu_plan_destroy(q), STRIX_SUCCESS);
+    };
+    submit(d, {"gemv_grouped_fused", "swiglu_rows"});
+    CHECK(fake::live.size() == live0);
+    submit(describe(g1, u1, 128), {"gemv_grouped", "swiglu_rows"});
+    CHECK(fake::live.size() == live0);
+    submit(describe(gate, other, I), {"gemv_fused", "gemv_fused", "moe_swiglu", "moe_swiglu", "moe_swiglu"});
+    strix_tp_swiglu_desc with_diag = d;
+    with_diag.diagnostic_gate = diag;
+    with_diag.diagnostic_up = diag + rows * H;
+    with_diag.diagnostic_bytes = rows * H * 4;
+    submit(with_diag, {"gemv_fused", "gemv_fused", "moe_swiglu", "moe_swiglu", "moe_swiglu"});
+
+    // A failed free keeps the plan; the weights go after it.
+    STATUS(strix_tp_swiglu_plan_create(c, &d, &st, &p), STRIX_SUCCESS);
+    fake::free_fail_at = 0;
+    STATUS(strix_tp_swiglu_plan_destroy(p), STRIX_ERROR_BACKEND);
+    STATUS(strix_weights_destroy(gate), STRIX_ERROR_INVALID_ARGUMENT);
+    STATUS(strix_tp_swiglu_plan_destroy(p), STRIX_SUCCESS);
+    for (strix_weights w : {gate, up, other, g1, u1}) STATUS(strix_weights_destroy(w), STRIX_SUCCESS);
+    for (void* q : {x, wide, diag}) CHECK(hipFree(q) == hipSuccess);
+    CHECK(fake::live.size() == live00);
+}
+
 int main() {
     policy_rules();
     pass_rules();
@@ -1026,6 +1134,7 @@ int main() {
     moe_reference_split_geometry(c, hs);
     noalloc_calls(c, hs);
     stream_read_calls(c, hs);
+    swiglu_plan(c, hs);
     // The default stream (NULL) is accepted everywhere a stream is.
     {
         const HostLinear L(128, 128, 2, false);

@@ -99,7 +99,26 @@ hipError_t launch_gemv_grouped(const DeviceWeights& g, const GroupWeights* table
     require(fake::in_live_block(c.x, xb), "grouped input outside device memory", "launch_gemv_grouped");
     require(fake::in_live_block(c.y, yb), "grouped output outside device memory", "launch_gemv_grouped");
     if (single_launch) check_state(g, c.rows, groups, *st, "launch_gemv_grouped");
+    const uint64_t need = gemv_workspace_bytes(g, uint32_t(c.rows)) * groups;
+    require(single_launch || !need || fake::in_live_block(c.workspace, need), "grouped workspace too small",
+            "launch_gemv_grouped");
+    // The activation: two groups of contiguous rows into a hidden view apart from them.
+    if (c.swiglu_hidden) {
+        const uint64_t hb = ((c.rows - 1) * c.swiglu_row_stride + g.output) * 4;
+        require(groups == 2 && c.y_row_stride == g.output && y_group_stride == c.rows * g.output,
+                "SwiGLU of two contiguous outputs", "launch_gemv_grouped");
+        require(c.swiglu_row_stride >= g.output && fake::in_live_block(c.swiglu_hidden, hb),
+                "hidden outside device memory", "launch_gemv_grouped");
+        auto meets = [&](const void* p, uint64_t bytes) {
+            const uintptr_t h = reinterpret_cast<uintptr_t>(c.swiglu_hidden), b = reinterpret_cast<uintptr_t>(p);
+            return h < b + bytes && b < h + hb;
+        };
+        require(!meets(c.x, xb) && !meets(c.y, yb), "hidden overlaps an operand", "launch_gemv_grouped");
+    }
     record(single_launch ? "gemv_grouped_fused" : "gemv_grouped", c.rows, c.workspace, nullptr, s, c.alpha, c.beta);
+    const hipError_t e = fake::launch_result();
+    if (e != hipSuccess || !c.swiglu_hidden) return e;
+    record("swiglu_rows", c.rows, nullptr, nullptr, s, 0, 0);
     return fake::launch_result();
 }
 
