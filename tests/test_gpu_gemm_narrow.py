@@ -73,6 +73,36 @@ def test_narrow_row_blocks(ctx, I, N, K, codebook, splits):
     w.destroy()
 
 
+@pytest.mark.parametrize("I,N,K,codebook", [(1024, 1152, 6, "mcg"), (1024, 1152, 8, "mul1")])
+def test_narrow_256_row_blocks(ctx, I, N, K, codebook):
+    """Several 256-row blocks (2 (N / 128) S workgroups per block, at least 512 in
+    all): whole, one row past a block, and a ragged last one, whose row tiles past
+    the rows read out of range; more than 4 bits take two loads per chunk."""
+    sizes = (769, 1024, 1025, 1300)
+    print(f"narrow gemm 256-row blocks {I}x{N} K={K} {codebook} M={sizes}", flush=True)
+    tr, suh, svh, b = synth.layer(I, N, K, 7200 + K, bias=True)
+    w = runtime.Weights(ctx, tr, suh, svh, b, codebook)
+    assert w.gemm_splits(16) == 8 and 2 * (N // 128) * 8 * ((769 + 255) // 256) >= 512
+    top = max(sizes)
+    x = torch.from_numpy(synth.activations(top, I, 7201)).to(DEV)
+    small = torch.empty((top, N), device=DEV)
+    for r in range(0, top, 128):   # 128-row blocks, one per call
+        part = torch.empty((min(128, top - r), N), device=DEV)
+        runtime.gemm(w, x[r:r + 128].contiguous(), part)
+        small[r:r + 128] = part
+    q = codec.dequantize_rotated(tr, K, codebook)
+    sel = np.r_[0:2, 254:258, 510:514, 766:770, 1022:1026, top - 2:top]
+    ref = linear.matmul_fp32_stages(x.cpu().numpy()[sel], tr, suh, svh, K, codebook, b, rotated=q)["output_fp32"]
+    for m in sizes:
+        y = torch.full((m + 1, N), float("nan"), device=DEV)   # one guard row
+        runtime.gemm(w, x[:m].contiguous(), y[:m])
+        assert torch.equal(_bits(y[:m]), _bits(small[:m])), m
+        assert bool(torch.isnan(y[m]).all())
+        rows = sel[sel < m]
+        synth.gate(y.cpu().numpy()[rows], ref[:len(rows)])
+    w.destroy()
+
+
 def test_narrow_passes(ctx):
     """A call whose planes pass 1 GiB runs in several passes, each row with the
     bits of a call of its own rows."""

@@ -1,16 +1,19 @@
-"""The routed-expert block's group list against its own route resolution.
+"""The routed-expert block's group list: against the oracle, and its down half
+against the route resolution of a down launch of its own.
 
-A submission's input launch lists the expert groups, which its gate/up and down
-launches read; a down launch of its own resolves the routes itself.  Both must
-give the same bits for any routes: shared and distinct experts, zero scores,
-tokens that are invalid (id outside the bank, repeated id, negative or
-non-finite score), one to 64 routes, a bank as small as one expert, and routes
-rewritten between submissions.
+The input launch ahead of every gate/up lists the expert groups, which gate/up
+and a submission's down read; a down launch of its own resolves the routes
+itself.  For any routes (shared and distinct experts, zero scores, tokens that
+are invalid by an id outside the bank, a repeated id, a negative or non-finite
+score, one to 64 routes, a bank as small as one expert, routes rewritten between
+submissions) hidden and the block output meet the block's bars against the staged
+FP32 oracle, and both downs give the same bits.
 """
 import numpy as np
 import pytest
 
 import synth
+from oracle import moe
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -57,7 +60,9 @@ def test_list_matches_own_resolution(ctx, E, rows, k):
     I, H = 512, 256
     bank = synth.moe_bank(E, I, H, 2, 9100 + E)
     ws = [tuple(runtime.Weights(ctx, *e[n][:4], "mul1") for n in ("gate", "up", "down")) for e in bank]
-    x = torch.from_numpy(synth.activations(rows, I, 9101)).to(DEV)
+    xh = synth.activations(rows, I, 9101)
+    x = torch.from_numpy(xh).to(DEV)
+    cache = {}
     ids = torch.zeros((rows, k), dtype=torch.int32, device=DEV)
     sc = torch.zeros((rows, k), device=DEV)
     y0, y1 = torch.empty((rows, I), device=DEV), torch.empty((rows, I), device=DEV)
@@ -71,6 +76,7 @@ def test_list_matches_own_resolution(ctx, E, rows, k):
         sc.copy_(torch.from_numpy(s))
         y0.fill_(7.0)
         y1.fill_(7.0)
+        listed.hidden.fill_(7.0)
         listed.submit()
         own.gate_up()
         own.down()
@@ -78,6 +84,21 @@ def test_list_matches_own_resolution(ctx, E, rows, k):
         assert torch.equal(y0.view(torch.int32), y1.view(torch.int32)), case
         if case == "invalid":
             assert bool(torch.isnan(y0).all())
+        got, hidden = y0.cpu().numpy(), listed.hidden.cpu().numpy().reshape(rows, k, H)
+        ref, href = moe.moe_block(xh, bank, i, s, cache=cache)
+        valid = moe.token_valid(i, s, E)
+        assert np.isnan(got[~valid]).all()
+        done = valid[:, None] & (s != 0)
+        assert (hidden[~done] == 7.0).all()   # no route but these is written
+        if done.any():
+            # hidden = SwiGLU of two projections: twice the single-linear bar; the
+            # down half from the device's own hidden: the single-linear gate; the
+            # three projections in a row: 1e-3 of the largest value
+            a, r = hidden[done].astype(np.float64), href[done].astype(np.float64)
+            assert np.max(np.abs(a - r)) <= 5e-4 * max(1.0, np.max(np.abs(r)))
+            assert np.sqrt(np.sum((a - r) ** 2) / np.sum(r ** 2)) <= 6e-5
+            synth.gate(got[valid], moe.down_combine(hidden, bank, i, s, cache=cache)[valid])
+            assert np.max(np.abs(got[valid] - ref[valid])) <= 1e-3 * np.max(np.abs(ref[valid]))
     for p in (listed, own):
         p.destroy()
     for e in ws:
