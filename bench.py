@@ -1,11 +1,12 @@
 """Benchmark of the EXL3 trellis hot path on one MI355X.
 
-Headline (`value`): decode GEMV, R = 1, K4 mul1, I = N = 4096 (the north-star
-configuration), through a prepared single-launch plan, as packed-weight GB/s
-over a cold rotation of >= 1 GiB of distinct weight copies (more than 4x the
-256 MB MALL), inputs resident in HBM.  One step = one GEMV call = one launch.
+Headline (`value`): decode GEMV, R = 1, K4 mul1, I = N = 4096, through a
+prepared single-launch plan, as packed-weight GB/s over a cold rotation of
+>= 1 GiB of distinct weight copies (more than 4x the 256 MB MALL), inputs
+resident in HBM.  One step = one GEMV call = one launch.
 
-Also reported on the same JSON line:
+Also reported on the same JSON line (the sweeps' cells in brief there, whole on
+stderr):
   sweep_gemv     decode GEMV, R = 1, 2, 4, 8 x {5120^2, 4096 -> 12288} x K4-6
   sweep_gemm     prefill GEMM, M = 128, 512, 2048 x the same shapes x K4-6
   grouped_o_a    16 groups x (4096 -> 1024) K5, R = 1..8, the split and the
@@ -27,7 +28,8 @@ the region, and the time per step is the timed region over the steps.  Every
 cell also reports median_pass_us, the median over 11 further whole passes
 (an event per pass), whatever --steps is.  Replayed outputs are checked
 bit-for-bit against an untimed eager call before the warm-up, after the timed
-region and after the passes (`replay_matches_eager`); the headline's output is
+region and after the passes (`replay_matches_eager`, of all the sweeps' cells
+`cells_replay_match_eager`); the headline's output is
 also checked against the NumPy oracle (reference GPU gate) before and after
 (`oracle_pass`, `oracle_maxabs`, `oracle_nrmse`).
 
@@ -527,7 +529,7 @@ def bench_moe(ctx, steps, warmup, seed):
 
 
 def cpu_baseline(sample_seconds=12.0):
-    """NumPy oracle (decode + staged FP32 layer) on the north-star layer, host cores.
+    """NumPy oracle (decode + staged FP32 layer) on the headline layer, host cores.
 
     Phases timed separately: (i) vectorized decode of the packed layer, (ii)
     the staged FP32 path from x to y given the decoded weights -- together the
@@ -734,6 +736,79 @@ def run_section(ctx, which, steps, warmup):
         print(json.dumps(c), flush=True)
 
 
+# What a sweep cell keeps on the result line.  Whoever reads the line may keep
+# only the last 16 KB of the output, which the full cells (up to 350 bytes
+# each) outgrow; they are printed whole on stderr as they are measured.
+BRIEF = ("groups", "experts", "distinct_experts", "M", "I", "N", "H", "K", "R", "rows", "top_k", "fold", "us",
+         "packed_GBps", "TFLOPs", "pct_fp16_peak", "pct_call_floor", "speedup_vs_fp16_library")
+
+
+def brief(cell):
+    return {k: cell[k] for k in BRIEF if k in cell}
+
+
+def result_line(head, ceil, cpu, sweep, gemm, grouped, moe_cell, warmup):
+    """The result line: the headline whole, the sweeps' cells in brief."""
+    import synth
+    ms = head["us"] / 1e3
+    achieved = head["packed_GBps"]
+    out = {
+        "metric": METRIC,
+        "value": head["packed_GBps"],
+        "unit": "GB/s",
+        "n_gpus": 1,
+        "steps": head["timed_steps"],
+        "warmup": warmup,
+        "ms_per_step": round(ms, 6),
+        "higher_is_better": True,
+        "scaling": "weak",
+        "vs_baseline": None,
+        "dtype": "u16 trellis decode -> fp16 operands, f32 accumulation",
+        "data": f"synthetic: PCG64 seed {synth.BASE_SEED} (+ section index) trellis/suh/svh/x",
+        "config": {"workload": "decode GEMV R1, EXL3 K4 mul1, I=N=4096, prepared single-launch plan, "
+                               f"cold rotation over {head['rotation_copies']} weight copies (>=1 GiB)",
+                   "us_per_call": head["us"], "median_pass_us": head["median_pass_us"], "passes": head["passes"],
+                   "warmup_launches": head["warmup_launches"],
+                   "pct_hbm_peak": head["pct_hbm_peak"], "pct_read_ceiling": head["pct_read_ceiling"],
+                   "replay_matches_eager": head["replay_matches_eager"],
+                   "oracle_pass": head["oracle_pass"], "oracle_maxabs": head["oracle_maxabs"],
+                   "oracle_nrmse": head["oracle_nrmse"],
+                   "call_floor_us": head["call_floor_us"], "call_floor_shape": head["call_floor_shape"],
+                   "pct_call_floor": head["pct_call_floor"], "read_ceiling_GBps": ceil["GBps"],
+                   "fp16_library_us": head["fp16_library_us"],
+                   "speedup_vs_fp16_library": head["speedup_vs_fp16_library"]},
+        "oracle_pass": head["oracle_pass"],
+        "oracle_maxabs": head["oracle_maxabs"],
+        "oracle_nrmse": head["oracle_nrmse"],
+        "oracle_gate": head.get("oracle_gate"),
+        "median_pass_us": head["median_pass_us"],
+        "read_ceiling": ceil,
+        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
+                     "frac": round(achieved / HBM_PEAK_GBPS, 4), "traffic": _traffic(),
+                     "kernel": HEADLINE_KERNEL, "algorithmic_bytes_per_launch": 4096 * 4096 * 4 // 8,
+                     "launch_us": head["us"], "median_pass_us": head["median_pass_us"],
+                     "read_ceiling_GBps": ceil["GBps"],
+                     "frac_of_read_ceiling": round(achieved / ceil["GBps"], 4),
+                     "call_floor_us": head["call_floor_us"]},
+        "cpu_baseline": cpu,
+        "cells_replay_match_eager": all(c["replay_matches_eager"]
+                                        for c in (*sweep, *gemm, *grouped, *([moe_cell] if moe_cell else ()))),
+        "sweep_gemv": [brief(c) for c in sweep],
+        "sweep_gemm": [brief(c) for c in gemm],
+        "grouped_o_a": [brief(c) for c in grouped],
+        "moe_k2": moe_cell and brief(moe_cell),
+    }
+    if gemm:
+        best, lib = {}, {}
+        for c in gemm:
+            if c["M"] == 2048:
+                best[f"{c['I']}x{c['N']} K{c['K']}"] = c["pct_fp16_peak"]
+                lib[f"{c['I']}x{c['N']}"] = c["fp16_library_pct_peak"]
+        out["prefill_m2048_pct_fp16_peak"] = best
+        out["prefill_m2048_fp16_library_pct_peak"] = lib
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -748,7 +823,7 @@ def main():
                     help="per-stage phase cycles of the M = 2048 GEMMs (instrumented library)")
     args = ap.parse_args()
     if args.gpus != 1:
-        print(f"bench.py measures one GPU only (every box here has one MI355X); --gpus {args.gpus} "
+        print(f"bench.py measures one GPU only; --gpus {args.gpus} "
               "is not supported", file=sys.stderr)
         sys.exit(2)
 
@@ -803,61 +878,7 @@ def main():
     cpu = None if args.no_cpu else cpu_baseline()
     if cpu:
         log(json.dumps(cpu))
-    ms = head["us"] / 1e3
-    achieved = head["packed_GBps"]
-    out = {
-        "metric": METRIC,
-        "value": head["packed_GBps"],
-        "unit": "GB/s",
-        "n_gpus": 1,
-        "steps": head["timed_steps"],
-        "warmup": args.warmup,
-        "ms_per_step": round(ms, 6),
-        "higher_is_better": True,
-        "scaling": "weak",
-        "vs_baseline": None,
-        "dtype": "u16 trellis decode -> fp16 operands, f32 accumulation",
-        "data": f"synthetic: PCG64 seed {synth.BASE_SEED} (+ config index) trellis/suh/svh/x per BASELINE configs",
-        "config": {"workload": "decode GEMV R1, EXL3 K4 mul1, I=N=4096, prepared single-launch plan, "
-                               f"cold rotation over {head['rotation_copies']} weight copies (>=1 GiB)",
-                   "us_per_call": head["us"], "median_pass_us": head["median_pass_us"], "passes": head["passes"],
-                   "warmup_launches": head["warmup_launches"],
-                   "pct_hbm_peak": head["pct_hbm_peak"], "pct_read_ceiling": head["pct_read_ceiling"],
-                   "replay_matches_eager": head["replay_matches_eager"],
-                   "oracle_pass": head["oracle_pass"], "oracle_maxabs": head["oracle_maxabs"],
-                   "oracle_nrmse": head["oracle_nrmse"],
-                   "call_floor_us": head["call_floor_us"], "call_floor_shape": head["call_floor_shape"],
-                   "pct_call_floor": head["pct_call_floor"], "read_ceiling_GBps": ceil["GBps"],
-                   "fp16_library_us": head["fp16_library_us"],
-                   "speedup_vs_fp16_library": head["speedup_vs_fp16_library"]},
-        "oracle_pass": head["oracle_pass"],
-        "oracle_maxabs": head["oracle_maxabs"],
-        "oracle_nrmse": head["oracle_nrmse"],
-        "oracle_gate": head.get("oracle_gate"),
-        "median_pass_us": head["median_pass_us"],
-        "read_ceiling": ceil,
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBPS, 4), "traffic": _traffic(),
-                     "kernel": HEADLINE_KERNEL, "algorithmic_bytes_per_launch": 4096 * 4096 * 4 // 8,
-                     "launch_us": head["us"], "median_pass_us": head["median_pass_us"],
-                     "read_ceiling_GBps": ceil["GBps"],
-                     "frac_of_read_ceiling": round(achieved / ceil["GBps"], 4),
-                     "call_floor_us": head["call_floor_us"]},
-        "cpu_baseline": cpu,
-        "sweep_gemv": sweep,
-        "sweep_gemm": gemm,
-        "grouped_o_a": grouped,
-        "moe_k2": moe_cell,
-    }
-    if gemm:
-        best, lib = {}, {}
-        for c in gemm:
-            if c["M"] == 2048:
-                best[f"{c['I']}x{c['N']} K{c['K']}"] = c["pct_fp16_peak"]
-                lib[f"{c['I']}x{c['N']}"] = c["fp16_library_pct_peak"]
-        out["prefill_m2048_pct_fp16_peak"] = best
-        out["prefill_m2048_fp16_library_pct_peak"] = lib
-    print(json.dumps(out), flush=True)
+    print(json.dumps(result_line(head, ceil, cpu, sweep, gemm, grouped, moe_cell, args.warmup)), flush=True)
 
 
 if __name__ == "__main__":
