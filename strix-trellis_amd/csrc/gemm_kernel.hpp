@@ -29,11 +29,11 @@
 //
 // Measured against 128 x 128 and 256 x 128 tiles of the same order (64 KiB of
 // LDS, two waves along each dimension; 320 workgroups on 5120^2 that multiplied
-// 128 rows whatever M was), calls, same bits: 5120^2 K5 M = 16 / 24 / 64 / 128 /
-// 200 24.5 / 24.6 / 27.6 / 30.9 / 40.7 -> 14.3 / 15.8 / 19.8 / 24.4 / 29.2 us, 4096
-// -> 12288 K6 29.1 / 29.4 / 32.0 / 35.7 / 49.7 -> 17.9 / 19.0 / 23.5 / 30.2 / 40.8 us,
-// 1152 -> 5120 K4 M = 16 / 128 25.0 / 30.3 -> 11.9 / 16.7 us; 5120 -> 1152 K4 M =
-// 512 / 4096 31.5 / 143.9 -> 27.0 / 127.9 us.
+// 128 rows whatever M was), prepared plans back to back on one buffer, same bits:
+// 5120^2 K5 M = 16 / 24 / 64 / 128 / 200 23.7 / 24.5 / 27.6 / 30.8 / 40.7 -> 13.6 /
+// 15.1 / 19.4 / 24.5 / 30.0 us, 4096 -> 12288 K6 29.0 / 29.4 / 32.1 / 35.8 / 50.4 ->
+// 16.6 / 18.6 / 23.9 / 31.1 / 41.9 us, 1152 -> 5120 K4 M = 16 / 128 25.2 / 30.2 ->
+// 11.8 / 16.5 us; 5120 -> 1152 K4 M = 512 / 4096 31.6 / 142.5 -> 24.8 / 120.6 us.
 //
 // MFMA 16x16x32 f16 operand layout (lane l, e = 0..7 / 0..3):
 //   A: A[l % 16][8 (l / 16) + e]      B: B[8 (l / 16) + e][l % 16]
@@ -88,6 +88,10 @@ __host__ __device__ __forceinline__ uint64_t afrag_offset(uint32_t rb, uint32_t 
 
 constexpr int NARROW_BSTAGE_BYTES = 4 * 4 * 64 * 16;   // 4 tiles x 4 K32 steps x 64 lanes x 16 B
 
+// Register budget: three workgroups per CU from 128 rows on (92-128 VGPRs at 128,
+// so four fit), four below.  The 256-row instances take 160-168 VGPRs, and at 6, 7
+// and 8 bits, whose chunks are longer, 1-10 more go to scratch (8-12, 20, 24-28
+// bytes per lane); M = 200 on 4096 -> 12288 K6 / K7 / K8 41.9 / 42.6 / 43.6 us.
 template <int K, int CB, int TM, bool FOLD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TM >= 8 ? 3 : 4)))
 void gemm_narrow_kernel(const uint32_t* trellis, const _Float16* afrag, uint32_t input,

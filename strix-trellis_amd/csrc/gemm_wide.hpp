@@ -10,9 +10,9 @@
 //     (buffer_load ... lds) from the 32x16 fragment-ordered workspace straight
 //     into LDS, two stages ahead (three buffers);
 //   * the weights (64 x BN = 4 input blocks x BN/16 tiles) are decoded from the
-//     trellis: wave w decodes one block's eight tiles, one chunk per lane,
-//     straight into 32x16 fragment order in LDS (double-buffered); the decode of
-//     stage st + 1 is interleaved with the MFMAs of stage st;
+//     trellis, one block's eight tiles per decoding wave, one chunk per lane,
+//     straight into 32x16 fragment order in LDS (double-buffered), by one half of
+//     the waves while the other half multiplies (the K loop below);
 //   * each wave multiplies its 128 output channels by its 64 (BN = 256) or 32
 //     (BN = 128) rows: 4 K16 steps x 4 x TM MFMAs.
 //
@@ -149,8 +149,14 @@ struct StageClock {
 // Each wave owns the 128 channels of one output H128 group and TM 32-row
 // blocks: BN = 256 as 4 (M) x 2 (N) waves of 64 rows, all eight decode;
 // BN = 128 as 8 (M) x 1 (N) waves of 32 rows, the stage's 8 tiles x 4 blocks
-// decoded by waves 0..3 (one per SIMD) while waves 4..7 issue empty chunk
-// loads so every wave counts the same vmcnt.
+// decoded by waves 0, 1 (early half) and 4, 5 (late half) while the others issue
+// empty chunk loads so every wave counts the same vmcnt.  Waves w and w + 4 share
+// a SIMD, so two SIMDs decode; decoders on all four (waves 0, 1, 6, 7) measured
+// from 1.6 % faster (K5) to 0.5 % slower (K4) over the layers that run these
+// tiles.  Against the loop in which waves 0..3 decoded beside their own MFMAs,
+// calls, K4, same bits: M = 512 on 2048^2 / 5120 -> 2304 31.5 / 38.2 -> 30.5 /
+// 36.6 us, M = 1024 on 5120 -> 1280 41.9 -> 40.4, M = 256 on 5120^2 38.4 -> 36.8
+// (28.8 / 33.8 / 37.3 / 34.0 with the present decode and epilogue).
 template <int K, int CB, int BN, bool HANDOFF>
 __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs a) {
     static_assert(!HANDOFF || BN == 256, "the handoff runs on 256 x 256 tiles");

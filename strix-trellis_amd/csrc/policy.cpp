@@ -113,14 +113,19 @@ uint64_t afrag_bytes(const DeviceWeights& w, uint64_t m) {
 // Column split and K split of a wide pass over the 256 CUs (one 512-thread
 // workgroup per CU).  `full` 256-column blocks run as 256 x 256 tiles, `half`
 // as 256 x 128 tiles, twice the workgroups at half the work each; a 256 x 128
-// tile takes ~0.8 of a 256 x 256 tile's time (the stage barrier and the A
-// stream do not shrink with it).  A pass whose tiles fill at most half the CUs
-// splits K (below), and there the full tiles win once eight splits or fewer
-// fill the CUs (tiles >= 32; measured on M = 256..768 of 5120^2 and 4096 ->
-// 12288, e.g. M = 512 on 4096 -> 12288: 110 -> 108 us, M = 256: 72 -> 64 us):
-// the plane traffic grows with S, so 20 tiles (M = 256 on 5120^2) stay half
-// tiles at half the split count.  A layer too short to split takes the half
-// tiles whenever all of them fit one wave of workgroups.
+// tile takes about two thirds of a 256 x 256 tile's time (256 whole tiles of 4096
+// -> 8192 at M = 2048 133 us, the same as 512 half tiles in two rounds 174): its
+// multiply slots are half as long, its decode slots, barriers and A stream are not.
+// A pass whose tiles fill at most half the CUs splits K (below).  There the plane
+// traffic grows with S, so with fewer than 32 tiles, where full ones would take
+// more than eight splits, half tiles at half the split count win (K4, full / half:
+// M = 512 on 2048^2 31.5 / 28.8 us, M = 1024 on 5120 -> 1280 40.6 / 37.3, M = 256
+// on 5120^2 36.5 / 34.0).  From 32 tiles on it is full ones: level at 40 (M = 512
+// on 5120^2 50.6 / 50.6), while at just 32 half tiles are ahead now (M = 1024 on
+// 2048^2 32.5 / 29.9; the line was drawn with an earlier loop, and moving it moves
+// the row classes of those calls).  A layer too short to split takes the half tiles
+// whenever all of them fit one round of workgroups (M = 512 on 512 -> 5120 23.5 /
+// 19.0 us, M = 1024 on 896 -> 4096 32.0 / 26.9).
 bool wide_can_split(const DeviceWeights& w) { return (w.input / 64) / kWideSplitMinStages >= 2; }
 WideSplit wide_split(uint64_t m, const DeviceWeights& w) {
     constexpr uint64_t kCus = 256;
