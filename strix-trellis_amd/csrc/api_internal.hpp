@@ -36,7 +36,7 @@ struct strix_weights_impl {
     uint64_t bytes = 0;
     uint64_t plans = 0;       // live plans retaining these weights
     // Single-launch state (planes, epochs, status) of plans created on these
-    // weights.  Graphs captured from a plan may replay after the plan is
+    // weights, and the gate and up rows of SwiGLU plans with these as the gate.  Graphs captured from a plan may replay after the plan is
     // destroyed, so the arrays live until the weights are destroyed, and
     // distinct plans never share one (the reference's rule for its completion
     // counters).
@@ -48,10 +48,12 @@ struct strix_weights_impl {
     std::vector<std::pair<void*, uint64_t>> idle_states;
 };
 
-// A single-launch state block held by a plan (base of a counter_arrays block).
+// A block of counter_arrays held by a plan; fresh: allocated for this plan, not
+// an idle one taken over.
 struct FusedBlock {
     void* base = nullptr;
     uint64_t bytes = 0;
+    bool fresh = false;
 };
 
 struct strix_linear_plan_impl {
@@ -154,6 +156,12 @@ stx::LinearCall to_call(const strix_matmul_desc& d, uint64_t rows, void* workspa
 // Enqueue the initial contents of a single-launch state of `bytes` at base:
 // status and epochs 0, every plane word GEMV_PLANE_EMPTY.
 hipError_t init_fused_state(void* base, uint64_t bytes, uint64_t planes_offset, hipStream_t hs);
+// A block of `bytes` owned by the weights: an idle one of that size if the
+// context lets plans take them, else a new one (contents undefined either way).
+strix_status hold_block(strix_weights w, uint64_t bytes, FusedBlock& block);
+// Undoes hold_block after a failed creation: a new block is freed, an idle one
+// is idle again.
+void discard_block(strix_weights w, FusedBlock& block);
 // Initialised single-launch GEMV state for `rows` rows on `w` (none when one
 // split suffices), owned by the weights: an idle block of the same size if
 // there is one, else a new one; the stream is synchronised.

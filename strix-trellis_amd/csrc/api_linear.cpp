@@ -8,6 +8,7 @@
 // descriptor; place_linear: workspace and device residence), then enqueued.
 // Plans run both steps once at creation and nothing but the device check at
 // submission.
+#include <algorithm>
 #include <new>
 
 #include "api_internal.hpp"
@@ -23,42 +24,50 @@ hipError_t init_fused_state(void* base, uint64_t bytes, uint64_t planes_offset, 
     return stx::launch_fill_u32(words + planes_offset / 4, stx::GEMV_PLANE_EMPTY, (bytes - planes_offset) / 4, hs);
 }
 
+strix_status hold_block(strix_weights w, uint64_t bytes, FusedBlock& block) {
+    block = {};
+    for (auto it = w->idle_states.begin(); w->owner->reuse_plan_state && it != w->idle_states.end(); ++it) {
+        if (it->second != bytes) continue;
+        block = {it->first, bytes, false};
+        w->idle_states.erase(it);
+        return STRIX_SUCCESS;
+    }
+    void* base = nullptr;
+    hipError_t e = hipMalloc(&base, bytes);
+    if (e != hipSuccess) return status_of(e);
+    try {
+        w->counter_arrays.push_back(base);   // released with the weights
+    } catch (...) {
+        (void)hipFree(base);
+        return STRIX_ERROR_OUT_OF_MEMORY;
+    }
+    block = {base, bytes, true};
+    return STRIX_SUCCESS;
+}
+
+void discard_block(strix_weights w, FusedBlock& block) {
+    if (!block.fresh) return release_fused_state(w, block);   // still owned by the weights; initialised again on reuse
+    const auto it = std::find(w->counter_arrays.begin(), w->counter_arrays.end(), block.base);
+    if (it != w->counter_arrays.end()) w->counter_arrays.erase(it);
+    (void)hipFree(block.base);
+    block = {};
+}
+
 strix_status make_fused_state(strix_weights w, uint64_t rows, hipStream_t hs, stx::FusedState& out,
                               FusedBlock& block) {
     out = {};
     block = {};
     const uint64_t bytes = stx::fused_state_bytes(w->dev, rows, 1);
     if (!bytes) return STRIX_SUCCESS;
-    void* state = nullptr;
-    bool reused = false;
-    for (auto it = w->idle_states.begin(); w->owner->reuse_plan_state && it != w->idle_states.end(); ++it) {
-        if (it->second == bytes) {
-            state = it->first;
-            w->idle_states.erase(it);
-            reused = true;
-            break;
-        }
-    }
-    hipError_t e = reused ? hipSuccess : hipMalloc(&state, bytes);
-    if (e == hipSuccess) e = init_fused_state(state, bytes, stx::fused_planes_offset(w->dev, 1), hs);
+    const strix_status s = hold_block(w, bytes, block);
+    if (s != STRIX_SUCCESS) return s;
+    hipError_t e = init_fused_state(block.base, bytes, stx::fused_planes_offset(w->dev, 1), hs);
     if (e == hipSuccess) e = hipStreamSynchronize(hs);
-    if (e == hipSuccess && !reused) {
-        try {
-            w->counter_arrays.push_back(state);   // released with the weights
-        } catch (...) {
-            e = hipErrorOutOfMemory;
-        }
-    }
     if (e != hipSuccess) {
-        FusedBlock back{state, bytes};
-        if (reused)
-            release_fused_state(w, back);   // still owned by the weights; initialised again on reuse
-        else if (state)
-            (void)hipFree(state);
+        discard_block(w, block);
         return status_of(e);
     }
-    block = {state, bytes};
-    out = stx::fused_state_at(state, w->dev, rows, 1);
+    out = stx::fused_state_at(block.base, w->dev, rows, 1);
     return STRIX_SUCCESS;
 }
 

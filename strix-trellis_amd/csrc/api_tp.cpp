@@ -21,8 +21,10 @@
 //     its activation launch.  5120 -> 1152 K4, 6 rows: 27.3 us in eight launches,
 //     11.2 us in two.
 // Workspaces: these plans keep their split partial planes in memory owned by
-// the weights (as linear plans do), so every workspace query returns 0 and a
-// caller workspace is optional.  Plans retain their weights.
+// the weights (as linear plans do; a SwiGLU plan's gate and up rows too, with
+// the gate), so every workspace query returns 0 and a caller workspace is
+// optional, and graphs captured from a plan may replay after it is destroyed.
+// Plans retain their weights.
 #include "api_internal.hpp"
 #include "moe.hpp"
 
@@ -45,14 +47,14 @@ struct strix_tp_dense_plan_impl {
     strix_context owner = nullptr;
     std::vector<TpMember> members;
     hipStream_t stream{};
-    // SwiGLU plans: gate/up outputs (diagnostic buffers or plan-owned scratch)
+    // SwiGLU plans: gate/up outputs (diagnostic buffers, or scratch owned by the gate's weights)
     // and the activation's destination.
     bool swiglu = false;
     float* gate = nullptr;
     float* up = nullptr;
     float* hidden = nullptr;
     uint64_t rows = 0, width = 0, hidden_stride = 0;
-    void* scratch = nullptr;
+    FusedBlock scratch{};
     // SwiGLU plans whose members run as one grouped launch: the table of their
     // weights and the single-launch state of two groups, in scratch.
     const stx::GroupWeights* table = nullptr;
@@ -146,7 +148,7 @@ GroupedScratch grouped_scratch(const stx::DeviceWeights& w, uint64_t rows) {
 strix_status arm_grouped(strix_tp_dense_plan_impl* p, hipStream_t hs) {
     const stx::DeviceWeights& w = p->members[0].weights->dev;
     const GroupedScratch g = grouped_scratch(w, p->rows);
-    char* base = static_cast<char*>(p->scratch);
+    char* base = static_cast<char*>(p->scratch.base);
     stx::GroupWeights table[2];
     for (int i = 0; i < 2; ++i) {
         const stx::DeviceWeights& m = p->members[i].weights->dev;
@@ -166,7 +168,7 @@ strix_status finish_create(Plan* p, strix_context c, hipStream_t hs) {
     strix_status s = p->table ? arm_grouped(p, hs) : arm(p->members, hs);
     if (s != STRIX_SUCCESS) {
         for (TpMember& m : p->members) release_fused_state(m.weights, m.block);
-        if (p->scratch) (void)hipFree(p->scratch);
+        if (p->scratch.base) discard_block(p->members[0].weights, p->scratch);
         delete p;
         return s;
     }
@@ -282,10 +284,7 @@ strix_status plan_destroy(strix_tp_dense_plan_impl* p) {
     if (!p) return STRIX_ERROR_INVALID_ARGUMENT;
     const strix_status s = on_context_device(p->owner);
     if (s != STRIX_SUCCESS) return s;
-    if (p->scratch) {
-        const hipError_t e = hipFree(p->scratch);
-        if (e != hipSuccess) return status_of(e);
-    }
+    if (p->scratch.base) release_fused_state(p->members[0].weights, p->scratch);
     for (TpMember& m : p->members) {
         release_fused_state(m.weights, m.block);
         --m.weights->plans;
@@ -458,15 +457,14 @@ strix_status strix_tp_swiglu_plan_create(strix_context c, const strix_tp_swiglu_
         p->gate = d->diagnostic_gate;
         p->up = d->diagnostic_up;
     } else {
-        const hipError_t e = hipMalloc(&p->scratch, grouped ? scratch.bytes : 2 * diag);
-        if (e != hipSuccess) {
+        if ((s = hold_block(d->gate, grouped ? scratch.bytes : 2 * diag, p->scratch)) != STRIX_SUCCESS) {
             delete p;
-            return e == hipErrorOutOfMemory ? STRIX_ERROR_OUT_OF_MEMORY : status_of(e);
+            return s;
         }
-        p->gate = static_cast<float*>(p->scratch);
+        p->gate = static_cast<float*>(p->scratch.base);
         p->up = p->gate + rows * H;
         if (grouped)
-            p->table = reinterpret_cast<const stx::GroupWeights*>(static_cast<char*>(p->scratch) + scratch.table);
+            p->table = reinterpret_cast<const stx::GroupWeights*>(static_cast<char*>(p->scratch.base) + scratch.table);
     }
     // Gate and up write contiguous [rows][H] F32 (the diagnostic layout).
     strix_tensor_desc gview{}, uview{};
@@ -499,7 +497,7 @@ strix_status strix_tp_swiglu_plan_create(strix_context c, const strix_tp_swiglu_
         }
     }
     if (s != STRIX_SUCCESS) {
-        if (p->scratch) (void)hipFree(p->scratch);
+        if (p->scratch.base) discard_block(d->gate, p->scratch);
         delete p;
         return s;
     }

@@ -1013,10 +1013,11 @@ static void stream_read_calls(strix_context c, hipStream_t hs) {
 }
 
 // SwiGLU plans: members of one rate and codebook are one grouped launch and one
-// activation launch on scratch that the plan owns; members of different rates,
-// and plans with diagnostic buffers, launch one by one.  A creation that fails
-// at any allocation, copy, fill or synchronisation leaves no allocation behind
-// and its weights free to go; submission is quiet; a plan keeps its weights.
+// activation launch; members of different rates, and plans with diagnostic
+// buffers, launch one by one.  A creation that fails at any allocation, copy,
+// fill or synchronisation leaves no allocation behind; submission is quiet; a
+// plan keeps its weights, and its rows and state outlive it with them (graphs
+// captured from it may replay), to be taken by later plans only on request.
 static void swiglu_plan(strix_context c, hipStream_t hs) {
     strix_stream st = stream_of(hs);
     const size_t live00 = fake::live.size();
@@ -1099,9 +1100,9 @@ static void swiglu_plan(strix_context c, hipStream_t hs) {
         STATUS(strix_tp_swiglu_plan_destroy(q), STRIX_SUCCESS);
     };
     submit(d, {"gemv_grouped_fused", "swiglu_rows"});
-    CHECK(fake::live.size() == live0);
+    CHECK(fake::live.size() == live0 + 1);   // one block, still there for its graphs
     submit(describe(g1, u1, 128), {"gemv_grouped", "swiglu_rows"});
-    CHECK(fake::live.size() == live0);
+    CHECK(fake::live.size() == live0 + 2);
     submit(describe(gate, other, I), {"gemv_fused", "gemv_fused", "moe_swiglu", "moe_swiglu", "moe_swiglu"});
     strix_tp_swiglu_desc with_diag = d;
     with_diag.diagnostic_gate = diag;
@@ -1109,12 +1110,27 @@ static void swiglu_plan(strix_context c, hipStream_t hs) {
     with_diag.diagnostic_bytes = rows * H * 4;
     submit(with_diag, {"gemv_fused", "gemv_fused", "moe_swiglu", "moe_swiglu", "moe_swiglu"});
 
-    // A failed free keeps the plan; the weights go after it.
+    // Without reuse the next plan gets a block of its own; with it, the idle one,
+    // initialised again (a failure there leaves it idle).
+    const size_t live1 = fake::live.size();
     STATUS(strix_tp_swiglu_plan_create(c, &d, &st, &p), STRIX_SUCCESS);
-    fake::free_fail_at = 0;
-    STATUS(strix_tp_swiglu_plan_destroy(p), STRIX_ERROR_BACKEND);
-    STATUS(strix_weights_destroy(gate), STRIX_ERROR_INVALID_ARGUMENT);
+    CHECK(fake::live.size() == live1 + 1);
     STATUS(strix_tp_swiglu_plan_destroy(p), STRIX_SUCCESS);
+    CHECK(fake::live.size() == live1 + 1);
+    STATUS(strix_amd_set_plan_state_reuse(c, 1), STRIX_SUCCESS);
+    fake::launch_fail_at = 1;
+    STATUS(strix_tp_swiglu_plan_create(c, &d, &st, &p), STRIX_ERROR_BACKEND);
+    fake::reset_failures();
+    CHECK(p == nullptr && fake::live.size() == live1 + 1);
+    for (int i = 0; i < 3; ++i) {
+        const fake::Counters before = fake::n;
+        STATUS(strix_tp_swiglu_plan_create(c, &d, &st, &p), STRIX_SUCCESS);
+        CHECK(fake::n.mallocs == before.mallocs && fake::live.size() == live1 + 1);
+        fake::launches.clear();
+        STATUS(strix_tp_swiglu_plan_submit(p), STRIX_SUCCESS);   // the fake checks the state it gets
+        STATUS(strix_tp_swiglu_plan_destroy(p), STRIX_SUCCESS);
+    }
+    STATUS(strix_amd_set_plan_state_reuse(c, 0), STRIX_SUCCESS);
     for (strix_weights w : {gate, up, other, g1, u1}) STATUS(strix_weights_destroy(w), STRIX_SUCCESS);
     for (void* q : {x, wide, diag}) CHECK(hipFree(q) == hipSuccess);
     CHECK(fake::live.size() == live00);

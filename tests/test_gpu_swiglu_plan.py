@@ -72,3 +72,33 @@ def test_swiglu_plan_forms(ctx, I, H, bits, codebooks, rows):
         p.destroy()
     for w in ws:
         w.destroy()
+
+
+def test_swiglu_graph_outlives_its_plan(ctx):
+    """Rows and state of a destroyed plan stay with the weights: a graph captured
+    from it replays with the same bits, and touches nothing allocated since."""
+    I, H, rows = 1024, 256, 3
+    print(f"swiglu graph after destroy {I}->{H} R={rows}", flush=True)
+    ws = [runtime.Weights(ctx, *synth.layer(I, H, 4, 8400 + i, bias=False), "mul1") for i in range(2)]
+    x = torch.from_numpy(synth.activations(rows, I, 8401)).to(DEV)
+    hidden, want = torch.empty((rows, H), device=DEV), torch.empty((rows, H), device=DEV)
+    g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    cap = runtime.TpSwigluPlan(*ws, x, hidden, stream=s)
+    with torch.cuda.graph(g, stream=s):
+        cap.submit()
+    cap.destroy()
+    others = [runtime.TpSwigluPlan(*ws, x, want) for _ in range(4)]   # the sizes a freed block would go to
+    guards = [torch.full((n,), 7.0, device=DEV) for n in (2048, 4096, 65536)]
+    for i in range(4):
+        x.copy_(torch.from_numpy(synth.activations(rows, I, 8402 + i)).to(DEV))
+        others[i].submit()
+        hidden.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(hidden.view(torch.int32), want.view(torch.int32))
+    assert all(bool((t == 7.0).all()) for t in guards)
+    for p in others:
+        p.destroy()
+    for w in ws:
+        w.destroy()
